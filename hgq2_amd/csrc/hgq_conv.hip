@@ -1524,6 +1524,17 @@ static int bwd_smallc_grid(const hgq_conv_geom &g) {
         else CALL(3, 3, 4); \
     } while (0)
 
+// A 1 x 1 convolution of unit stride without padding is a dense contraction over all pixels.
+static bool dense_shape(const hgq_conv_geom &g, int F) {
+    return g.kh == 1 && g.kw == 1 && g.sy == 1 && g.sx == 1 && g.py == 0 && g.px == 0 && g.OH == g.H && g.OW == g.W &&
+           gemm_parts_shape((int64_t)g.B * g.H * g.W, g.C, F);
+}
+// ... and its products run on the bf16-part kernels of hgq_gemm.hip unless the fp32 instruction was asked for
+static bool dense_parts(const hgq_conv_geom &g, int F) { return dense_shape(g, F) && hgq_dense_use_bf16_parts(-1) != 0; }
+static int64_t wgrad_slices(const hgq_conv_geom &g, int F, int64_t rows, const WgradCfg &c) {
+    return dense_shape(g, F) ? gemm_parts_splits(rows, g.C, F) : wgrad_splits(rows, c.n_kt * c.n_nt);
+}
+
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 template <int MODE>
@@ -1635,6 +1646,7 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
 #undef HGQ_SKINNY
         return check_launch("hgq_conv2d_fwd(few filters, long contraction)");
     }
+    if (nz == 1 && dense_parts(*g, F)) return gemm_parts_fwd(xq, qw, qb, y, rows, K, F, act, s);
     if (fwd_smallc_ok(*g, F)) {
         const int tiles_x = (g->OW + SC_TW - 1) / SC_TW, tiles_y = (g->OH + SC_TH - 1) / SC_TH;
         const dim3 grid((unsigned)persistent_grid((int64_t)g->B * tiles_x * tiles_y, 8));
@@ -1674,7 +1686,7 @@ extern "C" int64_t hgq_conv2d_bwd_workspace(const hgq_conv_geom *g, int F) {
     const int64_t rows = (int64_t)g->B * g->OH * g->OW;
     const int K = g->kh * g->kw * g->C;
     const WgradCfg c = wgrad_cfg(K, F);
-    int64_t slices = wgrad_splits(rows, c.n_kt * c.n_nt);
+    int64_t slices = wgrad_slices(*g, F, rows, c);
     if (bwd_smallc_ok(*g, F) && bwd_smallc_grid(*g) > slices) slices = bwd_smallc_grid(*g);
     if (conv_patch_wgrad_ok(*g, F) && conv_patch_wgrad_slices(*g, F) > slices) slices = conv_patch_wgrad_slices(*g, F);
     return slices * ((int64_t)K * F + F);
@@ -1695,7 +1707,7 @@ extern "C" int64_t hgq_conv2d_bwd_slice_count(const hgq_conv_geom *g, int F) {
     if (bwd_smallc_ok(*g, F)) return bwd_smallc_grid(*g);
     if (conv_patch_wgrad_ok(*g, F)) return conv_patch_wgrad_slices(*g, F);
     const WgradCfg c = wgrad_cfg(g->kh * g->kw * g->C, F);
-    return wgrad_splits(rows, c.n_kt * c.n_nt);
+    return wgrad_slices(*g, F, rows, c);
 }
 
 // reduce: the slices of the kernel / bias gradient are summed into dqw / dqb; otherwise they stay in `workspace`
@@ -1736,6 +1748,15 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
         if ((rc = check_launch("hgq_conv2d_bwd(few channels)"))) return rc;
         if (want_w && reduce) return reduce_parts(workspace, grid, KF + F, dqw, KF, dqb, (int64_t)F, nullptr, 0, s);
         return HGQ_OK;
+    }
+    if (dense_parts(*g, F)) {
+        const float *zmask = act == HGQ_ACT_RELU ? mask : nullptr;
+        if (dxq && (rc = gemm_parts_dgrad(dy, zmask, qw, dxq, rows, K, F, s))) return rc;
+        if (!dqw && !dqb) return HGQ_OK;
+        if (!workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
+        const int64_t splits = gemm_parts_splits(rows, K, F);
+        if ((rc = gemm_parts_wgrad(xq, dy, zmask, workspace, rows, K, F, splits, s))) return rc;
+        return reduce ? reduce_parts(workspace, (int)splits, KF + F, dqw, KF, dqb, (int64_t)F, nullptr, 0, s) : HGQ_OK;
     }
     if (dxq) {
         const int Kt = g->kh * g->kw * F;  // contraction length of the data gradient
@@ -1785,7 +1806,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
             return HGQ_OK;
         }
         const WgradCfg c = wgrad_cfg(K, F);
-        int64_t splits = wgrad_splits(rows, c.n_kt * c.n_nt);
+        int64_t splits = wgrad_slices(*g, F, rows, c);
         if (patch_shape) {
             if (splits > patch_slices) splits = patch_slices;
             if (splits < patch_slices && !reduce && (rc = fill_f32(workspace + splits * M, 0.f, (patch_slices - splits) * M, s))) return rc;

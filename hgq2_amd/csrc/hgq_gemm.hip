@@ -1,0 +1,397 @@
+// Contractions of dense layers beyond the streaming kernels' 64 x 64 (K or N > 64): forward, data gradient and weight
+// gradient as tiled matrix products on v_mfma_f32_32x32x16_bf16 over exact bf16 parts (hgq_device.h).
+//
+//   forward        Y[m, n]  = act(sum_k X[m, k] W[k, n] + b[n])
+//   data gradient  dX[m, k] = sum_n dZ[m, n] W[k, n]              dZ = dY where Y > 0 (ReLU), else dY
+//   weight grad.   dW[k, n] = sum_m X[m, k] dZ[m, n],  db[n] = sum_m dZ[m, n]      (split along m, one slice per split)
+//
+// An operand element is split into its parts ONCE per tile, on its way into LDS, where each part has a plane of its own with
+// eight consecutive contraction steps of a row in 16 bytes: an operand of the matrix instruction is one 128-bit LDS read.
+// (The implicit-GEMM kernels these replaced read their operands as single fp32 words - 32 LDS reads per instruction - and
+// split them again in every wavefront that multiplied by them.)
+// Planes that would be zero are neither written nor multiplied: the workgroup agrees on the number of parts of a tile step
+// from the low bits of its values (quantized operands of up to 8 bits: one part each, one matrix instruction per product);
+// gradients are arbitrary fp32 numbers and always take three.
+//
+// What bounds them: 50 000 x 256 onto 512 (153 MB, 13 GFLOP) takes 76 us, 50 000 x 512 onto 256 57 us (implicit GEMM: 174 and
+// 160 us) - 2 TB/s and 170 - 230 TFLOP/s, in between the two roofs: the chain load -> agree -> stage -> multiply of a tile step,
+// hidden by the second workgroup of a CU alone.  4096 x 256 x 512: forward 10.8, data gradient 15.9, weight gradient 13.4 us
+// (16.8, 25.5, 16.2 us).
+#include "hgq_device.h"
+#include "hgq_host.h"
+
+namespace hgq {
+
+enum { GP_FWD = 0, GP_DGRAD = 1, GP_WGRAD = 2 };
+
+// A load at voff + soff bytes; beyond the descriptor's range a lane gets zeros, dword by dword (soff counts towards the range).
+__device__ __forceinline__ f32x4_t gp_ld4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+__device__ __forceinline__ float gp_ld1(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+}
+
+struct GpArgs {
+    const float *a, *b;     // operands: FWD x, w; DGRAD dy, w; WGRAD x, dy
+    const float *mask;      // DGRAD / WGRAD: the forward output where the activation is a ReLU, else NULL
+    const float *bias;      // FWD
+    float *out;             // FWD / DGRAD [mo, no]; WGRAD slices [splits][mo * no + no]
+    int64_t rows;           // samples: FWD / DGRAD output rows, WGRAD contraction length
+    int64_t chunk;          // WGRAD: samples per split (a multiple of the contraction step)
+    int mo, no, kc;         // WGRAD: mo x no outputs; FWD / DGRAD: no output columns, kc contraction steps
+    int ntm, ntn;           // output tiles
+    int total;              // workgroups with work (tiles x splits)
+    int per_xcd;            // workgroups per XCD: consecutive ones (same rows, next columns) share an L2
+    int act;
+};
+
+// Staging of one operand tile of S rows (output index) x BK contraction steps by 256 threads.
+// KMAJOR = false: contraction steps are adjacent in memory: 128-bit loads (dword-aligned), four steps of a row each.
+// KMAJOR = true: output indices are adjacent in memory: a thread takes one output index and CPT consecutive steps, dword
+// loads that are whole cache lines per wavefront; it then holds what one 128-bit LDS write needs.  No alignment rule.
+template <int S, int BK, bool KMAJOR, bool MASKED>
+struct GpTile {
+    static constexpr int N = S * BK / 256;  // values per thread
+    static constexpr int LW = BK / 2 + 4;   // words per LDS row: 16-byte rows reads spread over all banks
+    static constexpr int QPR = BK / 4, RPP = 256 / QPR, NP = S / RPP;
+    float v[N], m[MASKED ? N : 1];
+
+    // base: the first element of the tile (row0 / step0 already applied by the caller), range in bytes from there
+    __device__ __forceinline__ void fetch(const float *base, const float *mbase, int64_t bytes, int ld, int cols_left, int step0) {
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(base, bytes), rm = buf_rsrc(MASKED && mbase ? mbase : base, MASKED && mbase ? bytes : 0);
+        const int tid = threadIdx.x;
+        if (KMAJOR) {
+            const int col = tid % S, grp = tid / S;
+            const uint32_t voff = col < cols_left ? (uint32_t)(grp * N * ld + col) * 4u : 0x80000000u;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                v[c] = gp_ld1(r, voff, (uint32_t)(c * ld) * 4u);
+                if (MASKED) m[c] = gp_ld1(rm, voff, (uint32_t)(c * ld) * 4u);
+            }
+        } else {
+            const int cq = tid % QPR, row = tid / QPR;
+            const uint32_t voff = (uint32_t)(row * ld + 4 * cq) * 4u;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const f32x4_t t = gp_ld4(r, voff, (uint32_t)(p * RPP * ld + step0) * 4u);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[4 * p + j] = t[j];
+                if (MASKED) {
+                    const f32x4_t u = gp_ld4(rm, voff, (uint32_t)(p * RPP * ld + step0) * 4u);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) m[4 * p + j] = u[j];
+                }
+            }
+        }
+    }
+    // steps past the end of the contraction read the next row: zeros instead (only the last tile step can hold any)
+    __device__ __forceinline__ void clip(int steps_left) {
+        if (!KMAJOR && steps_left < BK) {
+            const int c0 = 4 * (threadIdx.x % QPR);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (c0 + j >= steps_left) v[4 * p + j] = 0.f;
+            }
+        }
+    }
+    __device__ __forceinline__ void mask(bool on) {
+        if (MASKED && on) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) v[e] = m[e] > 0.f ? v[e] : 0.f;
+        }
+    }
+    __device__ __forceinline__ uint32_t low_bits() const {
+        uint32_t low = 0u;
+#pragma unroll
+        for (int e = 0; e < N; ++e) low |= __float_as_uint(v[e]);
+        return low;
+    }
+    // word index of this thread's unit u of four steps
+    __device__ __forceinline__ int at(int u) const {
+        const int tid = threadIdx.x;
+        if (KMAJOR) return (tid % S) * LW + (tid / S) * (N / 2) + 2 * u;
+        return (tid / QPR + RPP * u) * LW + 2 * (tid % QPR);
+    }
+    __device__ __forceinline__ void put(uint32_t *plane, const uint32_t (&w)[N / 2]) const {
+        if (KMAJOR && N % 8 == 0) {
+#pragma unroll
+            for (int u = 0; u < N / 8; ++u) *(u32x4_t *)(plane + at(2 * u)) = u32x4_t{w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]};
+        } else {
+#pragma unroll
+            for (int u = 0; u < N / 4; ++u) *(uint2 *)(plane + at(u)) = make_uint2(w[2 * u], w[2 * u + 1]);
+        }
+    }
+    // the first `parts` planes of the tile
+    __device__ __forceinline__ void stash(uint32_t *planes, int parts) const {
+        uint32_t w[N / 2];
+#pragma unroll
+        for (int e = 0; e < N; e += 2) w[e / 2] = bf16_pair(__float_as_uint(v[e]), __float_as_uint(v[e + 1]));
+        put(planes, w);
+        if (parts > 1) {
+            uint32_t l[N / 2];
+#pragma unroll
+            for (int e = 0; e < N; e += 2) {
+                uint32_t h0, m0, l0, h1, m1, l1;
+                bf16_parts(v[e], h0, m0, l0), bf16_parts(v[e + 1], h1, m1, l1);
+                w[e / 2] = bf16_pair(m0, m1), l[e / 2] = bf16_pair(l0, l1);
+            }
+            put(planes + S * LW, w);
+            if (parts > 2) put(planes + 2 * S * LW, l);
+        }
+    }
+};
+
+template <int OP, int BM, int BN, int BK>
+__global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
+    constexpr bool A_KMAJOR = OP == GP_WGRAD, B_KMAJOR = OP != GP_DGRAD;
+    constexpr int WN = BN >= 64 ? 2 : 1, WM = 4 / WN;    // wavefronts along the rows / columns of the tile
+    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;  // 32 x 32 blocks per wavefront
+    using TA = GpTile<BM, BK, A_KMAJOR, OP == GP_DGRAD>;
+    using TB = GpTile<BN, BK, B_KMAJOR, OP == GP_WGRAD>;
+    constexpr int LW = TA::LW;
+    __shared__ uint32_t as[3 * BM * LW], bs[3 * BN * LW], fl[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
+    const int t = (int)(blockIdx.x % 8u) * g.per_xcd + (int)(blockIdx.x / 8u);
+    if (t >= g.total || (int)(blockIdx.x / 8u) >= g.per_xcd) return;  // the whole workgroup
+    const int tile = OP == GP_WGRAD ? t % (g.ntm * g.ntn) : t, split = OP == GP_WGRAD ? t / (g.ntm * g.ntn) : 0;
+    const int mt = tile / g.ntn, nt = tile - mt * g.ntn;
+    const int64_t r0 = (int64_t)mt * BM;  // first output row
+    const int n0 = nt * BN;               // first output column
+    const bool relu = g.mask != nullptr;
+    // contraction range
+    const int64_t c_begin = OP == GP_WGRAD ? (int64_t)split * g.chunk : 0;
+    const int64_t c_end = OP == GP_WGRAD ? min(g.rows, c_begin + g.chunk) : (int64_t)g.kc;
+    const int n_steps = c_end > c_begin ? (int)((c_end - c_begin + BK - 1) / BK) : 0;
+
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx16{0};
+    TA ta;
+    TB tb;
+    float bsum = 0.f;
+    auto fetch = [&](int st) {
+        if (OP == GP_WGRAD) {
+            const int64_t m0 = c_begin + (int64_t)st * BK;
+            const int64_t left = c_end - m0;
+            ta.fetch(g.a + m0 * g.mo + r0, nullptr, (left * g.mo - r0) * 4, g.mo, g.mo - (int)r0, 0);
+            tb.fetch(g.b + m0 * g.no + n0, relu ? g.mask + m0 * g.no + n0 : nullptr, (left * g.no - n0) * 4, g.no, g.no - n0, 0);
+        } else {
+            const int64_t left = g.rows - r0;
+            ta.fetch(g.a + r0 * g.kc, relu ? g.mask + r0 * g.kc : nullptr, left * g.kc * 4, g.kc, 0, st * BK);
+            if (OP == GP_FWD) {
+                const int k0 = st * BK;
+                tb.fetch(g.b + (int64_t)k0 * g.no + n0, nullptr, ((int64_t)(g.kc - k0) * g.no - n0) * 4, g.no, g.no - n0, 0);
+            } else {
+                tb.fetch(g.b + (int64_t)n0 * g.kc, nullptr, (int64_t)(g.no - n0) * g.kc * 4, g.kc, 0, st * BK);
+            }
+        }
+    };
+    if (n_steps > 0) fetch(0);
+    for (int st = 0; st < n_steps; ++st) {
+        const int left = (int)min((int64_t)BK, c_end - c_begin - (int64_t)st * BK);
+        ta.clip(left), tb.clip(left);
+        ta.mask(relu), tb.mask(relu);
+        if (OP == GP_WGRAD) {
+            if (mt == 0) {
+#pragma unroll
+                for (int e = 0; e < TB::N; ++e) bsum += tb.v[e];
+            }
+        }
+        // how many parts the operands of this step have, agreed on by the workgroup: a word whose low half is zero is its
+        // own first part, one whose low byte is zero has at most two
+        uint32_t low_a = OP == GP_DGRAD ? 0u : ta.low_bits(), low_b = OP == GP_WGRAD ? 0u : tb.low_bits();
+        uint32_t f = 0u;
+        if (OP != GP_DGRAD) f |= (__any((low_a & 0xffffu) != 0u) ? 1u : 0u) | (__any((low_a & 0xffu) != 0u) ? 2u : 0u);
+        if (OP != GP_WGRAD) f |= (__any((low_b & 0xffffu) != 0u) ? 4u : 0u) | (__any((low_b & 0xffu) != 0u) ? 8u : 0u);
+        if (lane == 0) fl[wave] = f;
+        __syncthreads();  // the previous step's operand reads are over; the flags are there
+        f = (uint32_t)__builtin_amdgcn_readfirstlane((int)(fl[0] | fl[1] | fl[2] | fl[3]));
+        const int pa = OP == GP_DGRAD ? 3 : 1 + (int)(f & 1u) + (int)((f >> 1) & 1u);
+        const int pb = OP == GP_WGRAD ? 3 : 1 + (int)((f >> 2) & 1u) + (int)((f >> 3) & 1u);
+        ta.stash(as, pa), tb.stash(bs, pb);
+        __syncthreads();
+        if (st + 1 < n_steps) fetch(st + 1);
+        const int arow = wm * 32 * TM + (lane & 31), brow = wn * 32 * TN + (lane & 31), half = lane >> 5;
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ++ks) {
+            const uint32_t *ap = as + arow * LW + ks * 8 + half * 4, *bp = bs + brow * LW + ks * 8 + half * 4;
+            auto products = [&](const u32x4_t (&fa)[TM], const u32x4_t (&fb)[TN]) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] = mfma_bf16(fa[i], fb[j], acc[i][j]);
+            };
+            auto load_a = [&](u32x4_t (&fa)[TM], int p) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) fa[i] = *(const u32x4_t *)(ap + p * BM * LW + i * 32 * LW);
+            };
+            auto load_b = [&](u32x4_t (&fb)[TN], int p) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) fb[j] = *(const u32x4_t *)(bp + p * BN * LW + j * 32 * LW);
+            };
+            // the gradient's three parts against the parts of the quantized operand (or the parts of two quantized operands)
+            if (OP == GP_WGRAD) {
+                u32x4_t b0[TN], b1[TN], b2[TN];
+                load_b(b0, 0), load_b(b1, 1), load_b(b2, 2);
+                for (int p = 0; p < pa; ++p) {
+                    u32x4_t fa[TM];
+                    load_a(fa, p);
+                    products(fa, b0), products(fa, b1), products(fa, b2);
+                }
+            } else if (OP == GP_DGRAD) {
+                u32x4_t a0[TM], a1[TM], a2[TM];
+                load_a(a0, 0), load_a(a1, 1), load_a(a2, 2);
+                for (int p = 0; p < pb; ++p) {
+                    u32x4_t fb[TN];
+                    load_b(fb, p);
+                    products(a0, fb), products(a1, fb), products(a2, fb);
+                }
+            } else {
+                u32x4_t a0[TM], b0[TN];
+                load_a(a0, 0), load_b(b0, 0);
+                products(a0, b0);
+                for (int p = 1; p < pb; ++p) {
+                    u32x4_t fb[TN];
+                    load_b(fb, p);
+                    products(a0, fb);
+                }
+                for (int p = 1; p < pa; ++p) {
+                    u32x4_t fa[TM];
+                    load_a(fa, p);
+                    products(fa, b0);
+                    for (int q = 1; q < pb; ++q) {
+                        u32x4_t fb[TN];
+                        load_b(fb, q);
+                        products(fa, fb);
+                    }
+                }
+            }
+        }
+    }
+    // An infinity is not the sum of its bf16 parts (Inf - Inf) and a zero part turns it into a NaN: where a result is not
+    // finite the wavefront contracts its blocks again on the fp32 instruction, from memory.
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) < INFINITY);
+    if (__any(bad)) {
+        auto a_at = [&](int64_t i, int64_t c) -> float {  // output row i of the tile's matrix, contraction step c
+            if (c >= c_end || i >= (OP == GP_WGRAD ? (int64_t)g.mo : g.rows)) return 0.f;
+            const int64_t e = A_KMAJOR ? c * g.mo + i : i * g.kc + c;
+            return OP == GP_DGRAD && relu && !(g.mask[e] > 0.f) ? 0.f : g.a[e];
+        };
+        auto b_at = [&](int64_t j, int64_t c) -> float {
+            if (c >= c_end || j >= g.no) return 0.f;
+            const int64_t e = B_KMAJOR ? c * g.no + j : j * g.kc + c;
+            return OP == GP_WGRAD && relu && !(g.mask[e] > 0.f) ? 0.f : g.b[e];
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int64_t ai = r0 + wm * 32 * TM + i * 32 + (lane & 31), bj = n0 + wn * 32 * TN + j * 32 + (lane & 31);
+                floatx16 s = {0};
+                for (int64_t c = c_begin; c < c_end; c += 2)
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(a_at(ai, c + (lane >> 5)), b_at(bj, c + (lane >> 5)), s, 0, 0, 0);
+                acc[i][j] = s;
+            }
+    }
+    const int64_t out_rows = OP == GP_WGRAD ? (int64_t)g.mo : g.rows;
+    float *out = g.out + (OP == GP_WGRAD ? (int64_t)split * ((int64_t)g.mo * g.no + g.no) : 0);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int n = n0 + wn * 32 * TN + j * 32 + (lane & 31);
+        const float bv = (OP == GP_FWD && g.bias && n < g.no) ? g.bias[n] : 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t m = r0 + wm * 32 * TM + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                float v = acc[i][j][r];
+                if (OP == GP_FWD) {
+                    v += bv;
+                    if (g.act == HGQ_ACT_RELU) v = v > 0.f ? v : 0.f;
+                }
+                if (m < out_rows && n < g.no) out[m * g.no + n] = v;
+            }
+        }
+    }
+    if (OP == GP_WGRAD && mt == 0) {
+        // bias gradient: the threads of a column add up in a fixed order
+        float *red = (float *)bs;
+        __syncthreads();
+        red[tid] = bsum;
+        __syncthreads();
+        if (tid < BN && n0 + tid < g.no) {
+            float s = 0.f;
+#pragma unroll
+            for (int u = 0; u < 256 / BN; ++u) s += red[tid + u * BN];
+            out[(int64_t)g.mo * g.no + n0 + tid] = s;
+        }
+    }
+}
+
+template <int OP, int BM, int BN, int BK>
+static void gp_launch(GpArgs g, int splits, hipStream_t s) {
+    g.ntm = (int)(((OP == GP_WGRAD ? (int64_t)g.mo : g.rows) + BM - 1) / BM);
+    g.ntn = (g.no + BN - 1) / BN;
+    g.total = g.ntm * g.ntn * splits;
+    g.per_xcd = (g.total + 7) / 8;
+    hipLaunchKernelGGL((gemm_parts_kernel<OP, BM, BN, BK>), dim3((unsigned)g.per_xcd * 8u), dim3(256), 0, s, g);
+}
+
+// Tile of a product with `m` x `n` outputs.  128 x 128 tiles split and stage each operand value half as often, but a launch
+// needs two of them per CU to cover the staging of one with the products of the other; fewer outputs go to 64 x 64 tiles.
+template <int OP>
+static void gp_dispatch(const GpArgs &g, int64_t m, int64_t n, int splits, hipStream_t s) {
+    const int64_t big = ((m + 127) / 128) * ((n + 127) / 128) * splits;
+    if (n <= 32) gp_launch<OP, 128, 32, 32>(g, splits, s);
+    else if (big >= 384) gp_launch<OP, 128, 128, 32>(g, splits, s);
+    else gp_launch<OP, 64, 64, 64>(g, splits, s);
+}
+
+bool gemm_parts_shape(int64_t rows, int K, int N) {
+    return K >= 8 && N >= 1 && K <= (1 << 20) && N <= (1 << 20) && ((rows + 63) / 64) * (((int64_t)(K > N ? K : N) + 31) / 32) < (1ll << 30);
+}
+
+int64_t gemm_parts_splits(int64_t rows, int K, int N) {
+    const int64_t tiles = N <= 32 ? (K + 127) / 128 : (int64_t)((K + 63) / 64) * ((N + 63) / 64);
+    int64_t s = (512 + tiles - 1) / tiles;
+    const int64_t cap = N <= 32 ? (rows + 127) / 128 : (rows + 255) / 256;  // at least four tile steps each
+    if (s > cap) s = cap;
+    if (s > 512) s = 512;
+    return s < 1 ? 1 : s;
+}
+
+int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s) {
+    GpArgs g = {};
+    g.a = x, g.b = w, g.bias = bias, g.out = y, g.rows = rows, g.no = N, g.kc = K, g.act = act;
+    gp_dispatch<GP_FWD>(g, rows, N, 1, s);
+    return check_launch("gemm_parts(forward)");
+}
+
+int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, int64_t rows, int K, int N, hipStream_t s) {
+    GpArgs g = {};
+    g.a = dy, g.b = w, g.mask = mask, g.out = dx, g.rows = rows, g.no = K, g.kc = N;
+    gp_dispatch<GP_DGRAD>(g, rows, K, 1, s);
+    return check_launch("gemm_parts(data gradient)");
+}
+
+int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits, hipStream_t s) {
+    GpArgs g = {};
+    g.a = x, g.b = dy, g.mask = mask, g.out = part, g.rows = rows, g.mo = K, g.no = N;
+    g.chunk = ((rows + splits - 1) / splits + 63) / 64 * 64;
+    if (N <= 32) gp_launch<GP_WGRAD, 128, 32, 32>(g, (int)splits, s);
+    else gp_launch<GP_WGRAD, 64, 64, 64>(g, (int)splits, s);
+    return check_launch("gemm_parts(weight gradient)");
+}
+
+}  // namespace hgq

@@ -50,6 +50,15 @@ inline int fill_f32(float *p, float v, int64_t n, hipStream_t s) {
 int reduce_parts(const float *part, int n_parts, int64_t M, float *dqw, int64_t n_dqw, float *dqb, int64_t n_dqb, float *df,
                  int64_t n_df, hipStream_t s, float scale = 1.0f);
 
+// Dense contractions of any width on the bf16-part matrix instruction (hgq_gemm.hip): which shapes, the number of slices the
+// weight gradient leaves ([K N + N] each), and the three products.  mask: the forward output behind a ReLU, else NULL.
+bool gemm_parts_shape(int64_t rows, int K, int N);
+int64_t gemm_parts_splits(int64_t rows, int K, int N);
+int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s);
+int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, int64_t rows, int K, int N, hipStream_t s);
+int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits,
+                     hipStream_t s);
+
 // Convolution through LDS-resident operands (hgq_conv_patch.hip): mode 0 forward, 1 data gradient.
 bool conv_patch_ok(int mode, const hgq_conv_geom &g, int F);
 int conv_patch_launch(int mode, const float *src, const float *mask, const float *w, const float *bias, float *out,
