@@ -107,6 +107,8 @@ SIGNATURES = {
     'hgq_quantize_fwd_bwd': (c_int, [c_void_p] * 9 + [c_int64, c_int64, c_int64, c_int, c_void_p]),
     'hgq_quantize_fwd_multi': (c_int, [c_void_p, c_int, c_void_p]),
     'hgq_quantize_bwd_multi': (c_int, [c_void_p, c_int, c_void_p]),
+    'hgq_dense_stack_workspace': (c_int64, [c_void_p, c_int, c_int64]),
+    'hgq_dense_stack_predict': (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     'hgq_gdense_supported': (c_int, [c_int64, c_int, c_int, c_int]),
     'hgq_gdense_fwd': (c_int, [c_void_p] * 4 + [c_int64, c_int, c_int, c_int, c_int, c_void_p]),
     'hgq_gdense_bwd_workspace': (c_int64, [c_int64, c_int, c_int, c_int, c_int]),
@@ -177,6 +179,22 @@ class BitsDesc(ctypes.Structure):
 
     _fields_ = [('k', c_void_p), ('i', c_void_p), ('fb', c_void_p), ('size', c_int64), ('inner', c_int64), ('kbi', c_int),
                 ('add_mode', c_int), ('g_i', c_void_p), ('g_fb', c_void_p)]
+
+
+class StackQuant(ctypes.Structure):
+    """``hgq_stack_quant`` of include/hgq_hip.h."""
+
+    _fields_ = [('k', c_void_p), ('i', c_void_p), ('fb', c_void_p), ('size', c_int), ('inner', c_int), ('mode', c_int)]
+
+
+class StackLayer(ctypes.Structure):
+    """``hgq_stack_layer`` of include/hgq_hip.h."""
+
+    _fields_ = [('w', c_void_p), ('bias', c_void_p), ('kq', StackQuant), ('bq', StackQuant), ('iq', StackQuant),
+                ('K', c_int), ('N', c_int), ('act', c_int)]
+
+
+STACK_MAX_LAYERS = 8  # HGQ_STACK_MAX_LAYERS of include/hgq_hip.h
 
 
 class MlpLayer(ctypes.Structure):

@@ -366,8 +366,16 @@ class Sequential(Layer):
 
     def call(self, x, training=None):
         layers, k = list(self.layers), 0
+        predicts = training is False and not torch.is_grad_enabled()
+        if predicts:
+            from .layers.core._stack import predict_run
         while k < len(layers):
             layer = layers[k]
+            if predicts:
+                run = predict_run(layers, k, x)
+                if run is not None:
+                    x, k = run
+                    continue
             nxt = layers[k + 1] if k + 1 < len(layers) else None
             absorbs = getattr(layer, 'absorbs', None)
             if nxt is not None and absorbs is not None and isinstance(layer, Layer) and absorbs(nxt, x):

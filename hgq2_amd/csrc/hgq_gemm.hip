@@ -44,6 +44,7 @@ struct GpArgs {
     int total;              // workgroups with work (tiles x splits)
     int per_xcd;            // workgroups per XCD: consecutive ones (same rows, next columns) share an L2
     int act;
+    hgq_stack_quant oq;     // FWD: quantizer of the output's columns (oq.i NULL: none)
 };
 
 // Staging of one operand tile of S rows (output index) x BK contraction steps by 256 threads.
@@ -310,6 +311,13 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
     for (int j = 0; j < TN; ++j) {
         const int n = n0 + wn * 32 * TN + j * 32 + (lane & 31);
         const float bv = (OP == GP_FWD && g.bias && n < g.no) ? g.bias[n] : 0.f;
+        const bool quant = OP == GP_FWD && g.oq.i;
+        const Mode qm(g.oq.mode);
+        KIF qp = {0.f, 0.f, 0.f};
+        if (quant && n < g.no) {
+            const int e = g.oq.size == 1 ? 0 : n;
+            qp = resolve_kif(load_k(g.oq.k, e, qm.k_u8), g.oq.i[e], g.oq.fb[e], qm.kbi, qm.round_params);
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -319,6 +327,7 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
                 if (OP == GP_FWD) {
                     v += bv;
                     if (g.act == HGQ_ACT_RELU) v = v > 0.f ? v : 0.f;
+                    if (quant) v = quantize_dyn(v, qp, qm.round_mode, qm.overflow_mode, qm.training);
                 }
                 if (m < out_rows && n < g.no) out[m * g.no + n] = v;
             }
@@ -371,8 +380,10 @@ int64_t gemm_parts_splits(int64_t rows, int K, int N) {
     return s < 1 ? 1 : s;
 }
 
-int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s) {
+int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s,
+                   const hgq_stack_quant *oq) {
     GpArgs g = {};
+    if (oq) g.oq = *oq;
     g.a = x, g.b = w, g.bias = bias, g.out = y, g.rows = rows, g.no = N, g.kc = K, g.act = act;
     gp_dispatch<GP_FWD>(g, rows, N, 1, s);
     return check_launch("gemm_parts(forward)");

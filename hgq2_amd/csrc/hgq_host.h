@@ -54,7 +54,9 @@ int reduce_parts(const float *part, int n_parts, int64_t M, float *dqw, int64_t 
 // weight gradient leaves ([K N + N] each), and the three products.  mask: the forward output behind a ReLU, else NULL.
 bool gemm_parts_shape(int64_t rows, int K, int N);
 int64_t gemm_parts_splits(int64_t rows, int K, int N);
-int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s);
+// oq: a quantizer of the output's columns (one entry or N), applied behind the activation; NULL: none
+int gemm_parts_fwd(const float *x, const float *w, const float *bias, float *y, int64_t rows, int K, int N, int act, hipStream_t s,
+                   const hgq_stack_quant *oq = nullptr);
 int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, int64_t rows, int K, int N, hipStream_t s);
 int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits,
                      hipStream_t s);

@@ -1,0 +1,271 @@
+// Inference of a stack of QDense layers in one call: y = L_n(... L_1(x)), L(x) = act(q_in(x) q_w(W) + q_b(b)).
+//
+// Two forms.
+//
+// * Every width up to 64 (`stack_chain_kernel`): ONE launch.  A workgroup quantizes all kernels and biases into LDS, then
+//   takes tiles of 64 samples through every layer; between layers a tile stays in LDS and the next layer's input quantizer
+//   runs on the accumulator registers.  One event through 16-64-32-32-5 is bound by latency: four loads and one rounding
+//   per kernel entry, then a short matrix-instruction chain per layer; the call takes 75 us, most of it the host's (a launch
+//   per quantizer and contraction, sixteen in all: 512 us).
+// * Wider layers: one launch quantizes all kernels and biases into the workspace, one the input; then a tiled product per
+//   layer whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less per layer).
+//   50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and contraction: 484 us).
+//
+// Arithmetic per value is that of hgq_quantize_fwd and of the layer's own contraction; the variables are quantized again on
+// every call (they may have been written in between).
+#include "hgq_device.h"
+#include "hgq_host.h"
+
+namespace hgq {
+
+#define CHAIN_BM 64
+#define CHAIN_LD 65   // odd row stride: the 32 rows of an operand read fall into different banks
+#define CHAIN_LDS (160 * 1024)  // of a CU; seven layers of 64 x 64 fit
+#define CHAIN_NT 256  // four wavefronts: row half x column half of a tile
+
+struct ChainDev {
+    hgq_stack_layer l[HGQ_STACK_MAX_LAYERS];
+    int off_w[HGQ_STACK_MAX_LAYERS];  // kernel [Kp][Np], zero padded (Kp: multiple of 16, Np: of 32), then the bias [Np]
+    int n_layers, off_q, off_a;       // off_q: (k, i, f) of the input quantizers, [n_layers][3][64]; off_a: two tiles
+};
+
+__device__ __forceinline__ KIF stack_entry(const hgq_stack_quant &q, int e) {
+    const Mode m(q.mode);
+    return resolve_kif(load_k(q.k, e, m.k_u8), q.i[e], q.fb[e], m.kbi, m.round_params);
+}
+// bit-width entry of element e of a tensor with n elements
+__device__ __forceinline__ int stack_index(const hgq_stack_quant &q, int e, int n) {
+    return q.size == n ? e : (e / q.inner) % q.size;
+}
+__device__ __forceinline__ float stack_quantize(float v, const KIF &p, int mode) {
+    const Mode m(mode);
+    return quantize_dyn(v, p, m.round_mode, m.overflow_mode, m.training);
+}
+
+__global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d, const float *__restrict__ x, float *__restrict__ y,
+                                                               int64_t rows) {
+    extern __shared__ float lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int L = d.n_layers;
+    float *qt = lds + d.off_q, *tiles = lds + d.off_a;
+    for (int e = tid; e < d.off_a; e += CHAIN_NT) lds[e] = 0.f;
+    for (int e = tid; e < 2 * CHAIN_BM * CHAIN_LD; e += CHAIN_NT) tiles[e] = 0.f;
+    __syncthreads();
+    for (int l = 0; l < L; ++l) {
+        const hgq_stack_layer &h = d.l[l];
+        const int n = h.K * h.N, Np = (h.N + 31) & ~31, Kp = (h.K + 15) & ~15;
+        const FastDiv by_n((uint32_t)h.N);
+        float *w = lds + d.off_w[l];
+        for (int e0 = tid; e0 < n; e0 += 4 * CHAIN_NT) {
+            float v[4];
+            KIF p[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // (four entries in flight; the last trip repeats its own entry)
+                const int e = e0 + u * CHAIN_NT < n ? e0 + u * CHAIN_NT : e0;
+                v[u] = h.w[e];
+                p[u] = stack_entry(h.kq, stack_index(h.kq, e, n));
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = e0 + u * CHAIN_NT < n ? e0 + u * CHAIN_NT : e0;
+                const int k = (int)by_n.div((uint32_t)e);
+                w[k * Np + (e - k * h.N)] = stack_quantize(v[u], p[u], h.kq.mode);
+            }
+        }
+        if (h.bias && tid < h.N) w[Kp * Np + tid] = stack_quantize(h.bias[tid], stack_entry(h.bq, stack_index(h.bq, tid, h.N)), h.bq.mode);
+        if (h.iq.i && tid >= 64 && tid < 64 + h.K) {
+            const int c = tid - 64;
+            const KIF p = stack_entry(h.iq, h.iq.size == 1 ? 0 : c);
+            qt[l * 192 + c] = p.k, qt[l * 192 + 64 + c] = p.i, qt[l * 192 + 128 + c] = p.f;
+        }
+    }
+    __syncthreads();
+    const int64_t n_tiles = (rows + CHAIN_BM - 1) / CHAIN_BM;
+    const int K0 = d.l[0].K, NL = d.l[L - 1].N;
+    const FastDiv by_k0((uint32_t)K0), by_nl((uint32_t)NL);
+    const int rh = wave & 1, cb = wave >> 1, half = lane >> 5;
+    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        const int64_t r0 = tile * CHAIN_BM;
+        const int live = (int)(rows - r0 < CHAIN_BM ? rows - r0 : CHAIN_BM);
+        {
+            // the input tile: rows are contiguous; zeros past the last one (their results are not stored)
+            const __amdgpu_buffer_rsrc_t rs = buf_rsrc(x + r0 * K0, (int64_t)live * K0 * 4);
+            const bool quant = d.l[0].iq.i != nullptr;
+            for (int e0 = tid; e0 < CHAIN_BM * K0; e0 += 4 * CHAIN_NT) {
+                float v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = buf_ld1(rs, e0 + u * CHAIN_NT < CHAIN_BM * K0 ? (uint32_t)(e0 + u * CHAIN_NT) * 4u : BUF_OOB);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = e0 + u * CHAIN_NT;
+                    if (e < CHAIN_BM * K0) {
+                        const int row = (int)by_k0.div((uint32_t)e), c = e - row * K0;
+                        tiles[row * CHAIN_LD + c] = quant ? stack_quantize(v[u], KIF{qt[c], qt[64 + c], qt[128 + c]}, d.l[0].iq.mode) : v[u];
+                    }
+                }
+            }
+            // columns that pad the contraction to sixteen steps: a deeper layer of the previous tile has been here
+            const int pad = ((K0 + 15) & ~15) - K0;
+            for (int e = tid; e < CHAIN_BM * pad; e += CHAIN_NT) tiles[(e & (CHAIN_BM - 1)) * CHAIN_LD + K0 + e / CHAIN_BM] = 0.f;
+        }
+        for (int l = 0; l < L; ++l) {
+            const hgq_stack_layer &h = d.l[l];
+            const int Np = (h.N + 31) & ~31, batches = (h.K + 15) >> 4;
+            const float *src = tiles + (l & 1) * CHAIN_BM * CHAIN_LD;
+            float *dst = tiles + ((l + 1) & 1) * CHAIN_BM * CHAIN_LD;
+            const bool last = l + 1 == L;
+            __syncthreads();  // the source tile is complete
+            if (cb * 32 < Np) {
+                const float *w = lds + d.off_w[l];
+                const floatx16 zero = {0};
+                const floatx16 acc = mfma_chain_bf16<false, false>(zero, src + (rh * 32 + (lane & 31)) * CHAIN_LD + half, 1,
+                                                                   w + half * Np + cb * 32 + (lane & 31), Np, batches);
+                const int c = cb * 32 + (lane & 31);
+                const float b = w[batches * 16 * Np + c];
+                // the next layer's input quantizer, column c (nothing is read past its table: c < N = next K)
+                const bool quant = !last && d.l[last ? l : l + 1].iq.i != nullptr;
+                const int nm = d.l[last ? l : l + 1].iq.mode;
+                const float *qn = qt + (last ? 0 : l + 1) * 192;
+                const KIF p = {qn[c], qn[64 + c], qn[128 + c]};
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float v = acc[r] + b;
+                    if (h.act == HGQ_ACT_RELU) v = v > 0.f ? v : 0.f;
+                    if (quant) v = stack_quantize(v, p, nm);
+                    dst[(rh * 32 + (r >> 2) * 8 + half * 4 + (r & 3)) * CHAIN_LD + c] = c < h.N ? v : 0.f;
+                }
+            }
+        }
+        __syncthreads();
+        const float *out = tiles + (L & 1) * CHAIN_BM * CHAIN_LD;
+        for (int e = tid; e < live * NL; e += CHAIN_NT) {
+            const int row = (int)by_nl.div((uint32_t)e);
+            y[r0 * NL + e] = out[row * CHAIN_LD + (e - row * NL)];
+        }
+        __syncthreads();  // the next input tile goes into the first buffer
+    }
+}
+
+// All kernels and biases of a stack, quantized into the workspace.
+struct StackPrep {
+    hgq_stack_quant q[2 * HGQ_STACK_MAX_LAYERS];
+    const float *src[2 * HGQ_STACK_MAX_LAYERS];
+    float *dst[2 * HGQ_STACK_MAX_LAYERS];
+    int n[2 * HGQ_STACK_MAX_LAYERS];
+};
+__global__ __launch_bounds__(256) void stack_prep_kernel(const StackPrep p) {
+    const int it = blockIdx.y, n = p.n[it];
+    const hgq_stack_quant q = p.q[it];
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256)
+        p.dst[it][e] = stack_quantize(p.src[it][e], stack_entry(q, stack_index(q, e, n)), q.mode);
+}
+
+static bool quant_ok(const hgq_stack_quant &q, int64_t n) {
+    const Mode m(q.mode);
+    return q.k && q.i && q.fb && q.size >= 1 && q.inner >= 1 && n % ((int64_t)q.size * q.inner) == 0 && m.round_mode <= HGQ_RND_CONV &&
+           m.overflow_mode <= HGQ_SAT_SYM;
+}
+
+static int chain_layout(const hgq_stack_layer *layers, int n, ChainDev &d) {
+    int at = 0;
+    for (int l = 0; l < n; ++l) {
+        d.l[l] = layers[l];
+        d.off_w[l] = at;
+        at += (((layers[l].K + 15) & ~15) + 1) * ((layers[l].N + 31) & ~31);
+    }
+    d.n_layers = n;
+    d.off_q = at;
+    d.off_a = at + n * 192;
+    return (d.off_a + 2 * CHAIN_BM * CHAIN_LD) * (int)sizeof(float);
+}
+
+// 0: refused, 1: one launch, 2: a launch per layer
+static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
+    if (!layers || n < 1 || n > HGQ_STACK_MAX_LAYERS || rows < 1) return 0;
+    bool chain = true, wide = true;
+    for (int l = 0; l < n; ++l) {
+        const hgq_stack_layer &h = layers[l];
+        if (h.K < 1 || h.N < 1 || (int64_t)h.K * h.N > (1 << 26) || (l && h.K != layers[l - 1].N)) return 0;
+        if (!h.w || !quant_ok(h.kq, (int64_t)h.K * h.N) || (h.bias && !quant_ok(h.bq, h.N))) return 0;
+        if (h.iq.i && (!quant_ok(h.iq, h.K) || h.iq.inner != 1 || (h.iq.size != 1 && h.iq.size != h.K))) return 0;
+        chain = chain && h.K <= 64 && h.N <= 64;
+        wide = wide && gemm_parts_shape(rows, h.K, h.N);
+    }
+    ChainDev d;
+    if (chain && chain_layout(layers, n, d) <= CHAIN_LDS) return 1;
+    return (wide && hgq_dense_use_bf16_parts(-1) != 0) ? 2 : 0;
+}
+
+static int64_t image_floats(const hgq_stack_layer *layers, int n) {
+    int64_t at = 0;
+    for (int l = 0; l < n; ++l) at += ((int64_t)layers[l].K * layers[l].N + 3) / 4 * 4 + (layers[l].N + 3) / 4 * 4;
+    return at;
+}
+// widest tensor that goes into buffer `which` (0: inputs of even layers, 1: of odd layers)
+static int64_t buffer_floats(const hgq_stack_layer *layers, int n, int64_t rows, int which) {
+    int64_t w = 0;
+    for (int l = which; l < n; l += 2)
+        if ((l || layers[0].iq.i) && layers[l].K > w) w = layers[l].K;
+    return (w * rows + 3) / 4 * 4;
+}
+
+}  // namespace hgq
+
+using namespace hgq;
+
+extern "C" int64_t hgq_dense_stack_workspace(const hgq_stack_layer *layers, int n_layers, int64_t rows) {
+    const int form = stack_form(layers, n_layers, rows);
+    if (form != 2) return form == 1 ? 0 : -1;
+    return image_floats(layers, n_layers) + buffer_floats(layers, n_layers, rows, 0) + buffer_floats(layers, n_layers, rows, 1);
+}
+
+extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_layers, const float *x, float *y, int64_t rows,
+                                       float *workspace, void *stream) {
+    const int form = stack_form(layers, n_layers, rows);
+    if (!form) return fail(HGQ_ERR_UNSUPPORTED, "hgq_dense_stack_predict: these layers are not covered (ask hgq_dense_stack_workspace)");
+    if (!x || !y || (form == 2 && !workspace)) return fail(HGQ_ERR_ARG, "hgq_dense_stack_predict: null argument");
+    hipStream_t s = (hipStream_t)stream;
+    if (form == 1) {
+        ChainDev d = {};
+        const int bytes = chain_layout(layers, n_layers, d);
+        if (bytes > 64 * 1024) {
+            hipError_t e = hipFuncSetAttribute((const void *)stack_chain_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, CHAIN_LDS);
+            if (e != hipSuccess) return fail(HGQ_ERR_LAUNCH, "hgq_dense_stack_predict: hipFuncSetAttribute: %s", hipGetErrorString(e));
+        }
+        const int per_cu = CHAIN_LDS / bytes;  // each workgroup quantizes the kernels once: no more of them than fit at a time
+        const int grid = persistent_grid((rows + CHAIN_BM - 1) / CHAIN_BM, per_cu > 2 ? 2 : per_cu);
+        hipLaunchKernelGGL(stack_chain_kernel, dim3((unsigned)grid), dim3(CHAIN_NT), bytes, s, d, x, y, rows);
+        return check_launch("hgq_dense_stack_predict(chain)");
+    }
+    StackPrep p = {};
+    float *at = workspace, *qw[HGQ_STACK_MAX_LAYERS], *qb[HGQ_STACK_MAX_LAYERS];
+    int items = 0, most = 0;
+    for (int l = 0; l < n_layers; ++l) {
+        const hgq_stack_layer &h = layers[l];
+        const int n = h.K * h.N;
+        p.q[items] = h.kq, p.src[items] = h.w, p.dst[items] = qw[l] = at, p.n[items++] = n;
+        at += ((int64_t)n + 3) / 4 * 4;
+        if (n > most) most = n;
+        qb[l] = h.bias ? at : nullptr;
+        if (h.bias) p.q[items] = h.bq, p.src[items] = h.bias, p.dst[items] = at, p.n[items++] = h.N;
+        at += (h.N + 3) / 4 * 4;
+    }
+    const int gx = (most + 255) / 256 < 512 ? (most + 255) / 256 : 512;
+    hipLaunchKernelGGL(stack_prep_kernel, dim3((unsigned)gx, (unsigned)items), dim3(256), 0, s, p);
+    int rc = check_launch("hgq_dense_stack_predict(kernels)");
+    if (rc) return rc;
+    float *buf[2] = {at, at + buffer_floats(layers, n_layers, rows, 0)};
+    const float *cur = x;
+    if (const hgq_stack_quant &q = layers[0].iq; q.i) {
+        if ((rc = hgq_quantize_fwd(x, q.k, q.i, q.fb, buf[0], nullptr, nullptr, rows * layers[0].K, q.size, 1, q.mode, stream))) return rc;
+        cur = buf[0];
+    }
+    for (int l = 0; l < n_layers; ++l) {
+        const hgq_stack_layer &h = layers[l];
+        float *out = l + 1 == n_layers ? y : buf[(l + 1) & 1];
+        const hgq_stack_quant *oq = l + 1 < n_layers && layers[l + 1].iq.i ? &layers[l + 1].iq : nullptr;
+        if ((rc = gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq))) return rc;
+        cur = out;
+    }
+    return HGQ_OK;
+}

@@ -1,0 +1,116 @@
+"""Inference of consecutive QDense layers in one call of the library (``hgq_dense_stack_predict``): without gradients and
+outside training and tracing, a run of plain layers leaves no state behind, so nothing between them has to exist."""
+
+from __future__ import annotations
+
+import functools
+
+import torch
+
+from ... import _lib, ops
+from ...quantizer.internal import FixedPointQuantizerKBI, FixedPointQuantizerKIF
+from ...quantizer.internal.base import bw_layout
+from ...quantizer.quantizer import Quantizer
+from .dense import QDense
+
+_ACTS = {None: _lib.ACT_NONE, 'linear': _lib.ACT_NONE, 'relu': _lib.ACT_RELU}
+
+
+@functools.lru_cache(maxsize=1024)
+def _mode(round_mode, overflow_mode, training, kbi, symmetric):
+    return _lib.mode_bits(round_mode, overflow_mode, training=training, kbi=kbi, round_params=True, k_u8=True, symmetric=symmetric)
+
+
+def _describe(q, shape, device, out) -> bool:
+    """Fill ``out`` with the variables of the quantizer wrapper ``q`` as its call on a tensor of ``shape`` outside training
+    uses them; False where that call is anything but one deterministic fixed-point quantizer."""
+    if type(q) is not Quantizer or not q.built or not q.plain:
+        return False
+    fq = q.quantizer
+    kind = type(fq)
+    if kind is FixedPointQuantizerKIF:
+        kbi = False
+    elif kind is FixedPointQuantizerKBI:
+        kbi = True
+    else:
+        return False
+    if not fq.built or fq.stochastic or fq.__dict__.get('call') is not None:
+        return False
+    p = fq._parameters
+    i, fb, k = p.get('_i'), p.get('_b' if kbi else '_f'), fq._buffers.get('_var_k')
+    if k is not fq._k or k is None or i is None or fb is None or k.dtype is not torch.uint8 or i.dtype is not torch.float32 or fb.dtype is not torch.float32:
+        return False
+    if i.device != device or fb.device != device or k.device != device or not (i.is_contiguous() and fb.is_contiguous() and k.is_contiguous()):
+        return False
+    n = i.numel()
+    if fb.numel() != n or k.numel() != n:
+        return False
+    layout = bw_layout(i.shape, shape)
+    if layout is None or layout[0] != n:
+        return False
+    # a trainable WRAP quantizer of a weight rounds and does not wrap (`FixedPointQuantizerKIF.call`, `...KBI.call`)
+    rounds = fq._overflow_mode == 'WRAP' and fq.trainable and fq._is_weight and (not kbi or fq._round_mode == 'RND')
+    out.k, out.i, out.fb = k.data_ptr(), i.data_ptr(), fb.data_ptr()
+    out.size, out.inner = layout
+    out.mode = _mode(fq._round_mode, fq._overflow_mode, rounds, kbi, fq._symmetric)
+    return True
+
+
+def _layer(layer, rows, k_in, device, out) -> bool:
+    """Fill ``out`` for one layer; False where its call is more than quantize, contract, add, activate."""
+    if type(layer) is not QDense or not layer.built or layer._enable_oq or layer._act_name not in _ACTS or 'call' in layer.__dict__:
+        return False
+    w, b = layer._parameters.get('_kernel'), layer._parameters.get('bias')
+    if w is None or layer._kq is None or w.dim() != 2 or w.shape[0] != k_in or w.dtype is not torch.float32 or w.device != device or not w.is_contiguous():
+        return False
+    if not _describe(layer._kq, w.shape, device, out.kq):
+        return False
+    out.w, out.K, out.N, out.act = w.data_ptr(), k_in, w.shape[1], _ACTS[layer._act_name]
+    if b is not None:
+        if layer._bq is None or b.dtype is not torch.float32 or b.device != device or not b.is_contiguous() or b.numel() != out.N:
+            return False
+        if not _describe(layer._bq, b.shape, device, out.bq):
+            return False
+        out.bias = b.data_ptr()
+    if layer._enable_iq:
+        if not _describe(layer._iq, (rows, k_in), device, out.iq):
+            return False
+        size, inner = out.iq.size, out.iq.inner
+        if size == 1:
+            out.iq.inner = 1
+        elif size != k_in or inner != 1:
+            return False
+    return True
+
+
+def _ordinary_call() -> bool:
+    """No tracer, transform, dual level or mode wants to see the operators of this call."""
+    return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch.jit.is_tracing()
+                or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def predict_run(layers, first, x):
+    """``(output, index behind the last layer taken)`` for the longest run of layers from ``first`` on that one library call
+    covers, or ``None``."""
+    if type(x) is not torch.Tensor or not x.is_cuda or x.dtype is not torch.float32 or x.dim() != 2 or not x.numel() or not _ordinary_call():
+        return None
+    rows, width = x.shape
+    descs = (_lib.StackLayer * _lib.STACK_MAX_LAYERS)()
+    n, device = 0, x.device
+    if rows > 2**30 or device.index != torch.cuda.current_device():
+        return None
+    while n < _lib.STACK_MAX_LAYERS and first + n < len(layers):
+        if not _layer(layers[first + n], rows, width, device, descs[n]):
+            break
+        width = descs[n].N
+        n += 1
+    if n == 0:
+        return None
+    y = ops.dense_stack_predict(x, descs, n, width)
+    if y is None:
+        return None
+    for layer in layers[first:first + n]:
+        layer._losses = []
+        layer._deferred, layer._oq_applied_in_call = None, False
+    return y, first + n

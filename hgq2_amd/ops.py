@@ -2603,6 +2603,23 @@ def matmul_bias_act(x2d: Tensor, qw: Tensor, qb, act: int = 0) -> Tensor:
     return y.view(rows, N)
 
 
+def dense_stack_predict(x, descs, n: int, n_out: int):
+    """Output ``[rows, n_out]`` of a stack of dense layers described by the first ``n`` entries of ``descs``
+    (``_lib.StackLayer``) without gradients, or ``None`` where the library does not cover it."""
+    lib = _lib.load()
+    rows = x.shape[0]
+    floats = lib.hgq_dense_stack_workspace(descs, n, rows)
+    if floats < 0:
+        return None
+    if not x.is_contiguous():
+        x = x.contiguous()
+    y = torch.empty((rows, n_out), dtype=torch.float32, device=x.device)
+    ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
+    _lib.check(lib.hgq_dense_stack_predict(descs, n, x.data_ptr(), y.data_ptr(), rows, ws.data_ptr() if floats else None, _stream()),
+               'hgq_dense_stack_predict')
+    return y
+
+
 class _ColMoments(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):

@@ -205,6 +205,28 @@ typedef struct {
 int hgq_quantize_fwd_multi(const hgq_quant_item *items, int count, void *stream);
 int hgq_quantize_bwd_multi(const hgq_quant_grad_item *items, int count, void *stream);
 
+/*
+ * Inference of a stack of QDense layers (the composition of QDense.call with training=False,
+ * src/hgq/layers/core/dense.py:72-79): y [rows, N_last] from x [rows, K_first].  Every quantizer comes as its raw variables;
+ * element e of the quantized tensor uses entry (e / inner) % size of them.  Input quantizers: one entry, or one per column
+ * (inner 1); iq.i == NULL: none.  bias == NULL: none.  act: HGQ_ACT_*.  A layer's K is the previous one's N.
+ * hgq_dense_stack_workspace: floats of scratch (16-byte aligned), 0 when none is needed, -1 when the call is not covered.
+ */
+#define HGQ_STACK_MAX_LAYERS 8
+typedef struct {
+    const void *k;
+    const float *i, *fb;
+    int size, inner, mode;
+} hgq_stack_quant;
+typedef struct {
+    const float *w, *bias;
+    hgq_stack_quant kq, bq, iq;
+    int K, N, act;
+} hgq_stack_layer;
+int64_t hgq_dense_stack_workspace(const hgq_stack_layer *layers, int n_layers, int64_t rows);
+int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_layers, const float *x, float *y, int64_t rows,
+                            float *workspace, void *stream);
+
 int hgq_quantize_bwd(const float *dy, const float *x, const void *k, const float *i, const float *fb,
                      float *dx, float *di, float *dfb, int64_t n, int64_t bw_size, int64_t bw_inner,
                      int mode, void *stream);
