@@ -202,9 +202,12 @@ __global__ __launch_bounds__(HGQ_EBOPS_NT) void dense_ebops_multi_kernel(DenseEb
 
 // Mean squared error: per-workgroup partial sums (fixed order inside a workgroup), added in order
 // by one wavefront of a second launch: the loss does not depend on scheduling.
-#define MSE_PARTS 1024
+#define MSE_PARTS 2048
 // dpred (may be null): also receives the gradient for a unit upstream gradient, (pred - target) * two_over_n, the value
 // mse_bwd_kernel gives for g = 1
+// NT: operands beyond the 256 MB memory-side cache, which the next launch could not find there anyway.  805 MB (67 Mi values): 154 us =
+// 5.2 TB/s, what streams of this size reach on this card (four workgroups per CU, cached: 170 us).
+template <bool NT>
 __global__ __launch_bounds__(256) void mse_partial_kernel(const float *__restrict__ pred, const float *__restrict__ target, int64_t n,
                                                           float *__restrict__ part, float *__restrict__ dpred, float two_over_n) {
     __shared__ float red[4];
@@ -216,14 +219,17 @@ __global__ __launch_bounds__(256) void mse_partial_kernel(const float *__restric
         f32x4_t p[4], t[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            p[u] = ((const f32x4_t *)pred)[i + u * stride];
-            t[u] = target ? ((const f32x4_t *)target)[i + u * stride] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+            p[u] = NT ? __builtin_nontemporal_load((const f32x4_t *)pred + i + u * stride) : ((const f32x4_t *)pred)[i + u * stride];
+            t[u] = !target ? f32x4_t{0.f, 0.f, 0.f, 0.f}
+                   : NT    ? __builtin_nontemporal_load((const f32x4_t *)target + i + u * stride)
+                           : ((const f32x4_t *)target)[i + u * stride];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const f32x4_t d = p[u] - t[u];
             acc += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
-            if (dpred) ((f32x4_t *)dpred)[i + u * stride] = d * two_over_n;
+            if (dpred && NT) __builtin_nontemporal_store(d * two_over_n, (f32x4_t *)dpred + i + u * stride);
+            else if (dpred) ((f32x4_t *)dpred)[i + u * stride] = d * two_over_n;
         }
     }
     for (; i < n4; i += stride) {
@@ -243,11 +249,18 @@ __global__ __launch_bounds__(256) void mse_partial_kernel(const float *__restric
     if (threadIdx.x == 0) part[blockIdx.x] = acc;
 }
 
-__global__ __launch_bounds__(64) void mse_finish_kernel(const float *__restrict__ part, int n_parts, float inv_n, float *loss) {
-    float acc = 0.f;
-    for (int i = threadIdx.x; i < n_parts; i += 64) acc += part[i];
+__global__ __launch_bounds__(256) void mse_finish_kernel(const float *__restrict__ part, int n_parts, float inv_n, float *loss) {
+    __shared__ float red[4];
+    float v[MSE_PARTS / 256], acc = 0.f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    for (int u = 0; u < MSE_PARTS / 256; ++u) {
+        const int i = u * 256 + threadIdx.x;
+        v[u] = part[i < n_parts ? i : 0];
+        v[u] = i < n_parts ? v[u] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < MSE_PARTS / 256; ++u) acc += v[u];
+    acc = block_sum_256(acc, red);
     if (threadIdx.x == 0) loss[0] = acc * inv_n;
 }
 
@@ -920,12 +933,12 @@ extern "C" int hgq_mse_fwd(const float *pred, const float *target, float *loss, 
     if (!pred || !loss || !workspace) return fail(HGQ_ERR_ARG, "hgq_mse_fwd: null pointer");
     if (((uintptr_t)pred & 15u) || ((uintptr_t)target & 15u)) return fail(HGQ_ERR_ARG, "hgq_mse_fwd: operands must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
-    int grid = persistent_grid(((n >> 2) + 255) / 256, 4);
+    int grid = persistent_grid(((n >> 2) + 255) / 256, 8);
     if (grid > MSE_PARTS) grid = MSE_PARTS;
-    hipLaunchKernelGGL(mse_partial_kernel, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, (float *)nullptr, 0.f);
+    hipLaunchKernelGGL(mse_partial_kernel<false>, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, (float *)nullptr, 0.f);
     int rc = check_launch("hgq_mse_fwd");
     if (rc) return rc;
-    hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(64), 0, s, workspace, grid, 1.0f / (float)n, loss);
+    hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(256), 0, s, workspace, grid, 1.0f / (float)n, loss);
     return check_launch("hgq_mse_fwd(finish)");
 }
 
@@ -935,12 +948,15 @@ extern "C" int hgq_mse_fwd_bwd(const float *pred, const float *target, float *lo
     if (((uintptr_t)pred & 15u) || ((uintptr_t)target & 15u) || ((uintptr_t)dpred & 15u))
         return fail(HGQ_ERR_ARG, "hgq_mse_fwd_bwd: operands must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
-    int grid = persistent_grid(((n >> 2) + 255) / 256, 4);
+    int grid = persistent_grid(((n >> 2) + 255) / 256, 8);
     if (grid > MSE_PARTS) grid = MSE_PARTS;
-    hipLaunchKernelGGL(mse_partial_kernel, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, dpred, 2.0f / (float)n);
+    if (n > (1 << 24))
+        hipLaunchKernelGGL(mse_partial_kernel<true>, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, dpred, 2.0f / (float)n);
+    else
+        hipLaunchKernelGGL(mse_partial_kernel<false>, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, dpred, 2.0f / (float)n);
     int rc = check_launch("hgq_mse_fwd_bwd");
     if (rc) return rc;
-    hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(64), 0, s, workspace, grid, 1.0f / (float)n, loss);
+    hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(256), 0, s, workspace, grid, 1.0f / (float)n, loss);
     return check_launch("hgq_mse_fwd_bwd(finish)");
 }
 
