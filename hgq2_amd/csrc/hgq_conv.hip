@@ -1662,6 +1662,7 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
 #undef HGQ_FWD_SC
         return check_launch("hgq_conv2d_fwd(few channels)");
     }
+    if (nz == 1 && conv_thin_fwd_ok(*g, F)) return conv_thin_fwd(xq, qw, qb, y, *g, F, act, s);
     if (nz == 1 && aligned16(xq) && conv_patch_ok(0, *g, F)) return conv_patch_launch(0, xq, nullptr, qw, qb, y, *g, F, act, s);
     const bool vec = g->C % 4 == 0 && aligned16(xq) && (int64_t)g->B * g->H * g->W * g->C * 4 < (1ll << 31);
     if (F <= 32) {
@@ -1688,6 +1689,7 @@ extern "C" int64_t hgq_conv2d_bwd_workspace(const hgq_conv_geom *g, int F) {
     const WgradCfg c = wgrad_cfg(K, F);
     int64_t slices = wgrad_slices(*g, F, rows, c);
     if (bwd_smallc_ok(*g, F) && bwd_smallc_grid(*g) > slices) slices = bwd_smallc_grid(*g);
+    if (conv_thin_bwd_ok(*g, F) && conv_thin_slices(*g) > slices) slices = conv_thin_slices(*g);
     if (conv_patch_wgrad_ok(*g, F) && conv_patch_wgrad_slices(*g, F) > slices) slices = conv_patch_wgrad_slices(*g, F);
     return slices * ((int64_t)K * F + F);
 }
@@ -1704,6 +1706,7 @@ extern "C" int64_t hgq_conv2d_bwd_slice_count(const hgq_conv_geom *g, int F) {
     if (check_geom(g, F, "hgq_conv2d_bwd_slice_count")) return -1;
     const int64_t rows = (int64_t)g->B * g->OH * g->OW;
     if (rows == 0) return 1;
+    if (conv_thin_bwd_ok(*g, F)) return conv_thin_slices(*g);
     if (bwd_smallc_ok(*g, F)) return bwd_smallc_grid(*g);
     if (conv_patch_wgrad_ok(*g, F)) return conv_patch_wgrad_slices(*g, F);
     const WgradCfg c = wgrad_cfg(g->kh * g->kw * g->C, F);
@@ -1734,6 +1737,12 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
     const float *mask = (act == HGQ_ACT_RELU || dyp) ? y : nullptr;
     if (dyp && !(hgq_conv2d_maxpool_bwd_supported(g, F) && aligned16(dyp) && (code ? ((uintptr_t)code & 3u) == 0 : aligned16(y))))
         return fail(HGQ_ERR_UNSUPPORTED, "hgq_conv2d_maxpool_bwd: shape or alignment not supported (ask hgq_conv2d_maxpool_bwd_supported)");
+    if (conv_thin_bwd_ok(*g, F)) {
+        const bool want_w = dqw || dqb;
+        if (want_w && !workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
+        if ((rc = conv_thin_bwd(dy, mask, dyp, code, xq, qw, dxq, want_w ? workspace : nullptr, *g, F, act, s))) return rc;
+        return want_w && reduce ? reduce_parts(workspace, conv_thin_slices(*g), KF + F, dqw, KF, dqb, (int64_t)F, nullptr, 0, s) : HGQ_OK;
+    }
     if (bwd_smallc_ok(*g, F)) {
         const bool want_w = dqw || dqb;
         if (want_w && !workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");

@@ -61,6 +61,15 @@ int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *
 int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits,
                      hipStream_t s);
 
+// Convolutions over few input values per pixel (hgq_conv_thin.hip): which shapes, the slices the backward pass leaves
+// ([K F + F] each), forward, and data + weight + bias gradient in one pass.
+bool conv_thin_fwd_ok(const hgq_conv_geom &g, int F);
+bool conv_thin_bwd_ok(const hgq_conv_geom &g, int F);
+int conv_thin_slices(const hgq_conv_geom &g);
+int conv_thin_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);
+int conv_thin_bwd(const float *dy, const float *mask, const float *dyp, const uint8_t *code, const float *x, const float *w, float *dx,
+                  float *part, const hgq_conv_geom &g, int F, int act, hipStream_t s);
+
 // Convolution through LDS-resident operands (hgq_conv_patch.hip): mode 0 forward, 1 data gradient.
 bool conv_patch_ok(int mode, const hgq_conv_geom &g, int F);
 int conv_patch_launch(int mode, const float *src, const float *mask, const float *w, const float *bias, float *out,
