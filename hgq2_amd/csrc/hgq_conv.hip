@@ -1531,8 +1531,12 @@ static bool dense_shape(const hgq_conv_geom &g, int F) {
 }
 // ... and its products run on the bf16-part kernels of hgq_gemm.hip unless the fp32 instruction was asked for
 static bool dense_parts(const hgq_conv_geom &g, int F) { return dense_shape(g, F) && hgq_dense_use_bf16_parts(-1) != 0; }
+// The tiled product gathers the weight gradient's source element by element, for any depth; where four channels make a 128-bit
+// gather wgrad_vec_kernel is the faster one (300 x 11 x 11, 3 x 3, 40 -> 40: 21 against 38 us; 1024 x 13 x 13, 37 -> 37: all
+// gradients 382 -> 220 us with the tiled product).
+static bool wgrad_parts(const hgq_conv_geom &g, int F) { return g.C % 4 != 0 && conv_parts_shape(g, F); }
 static int64_t wgrad_slices(const hgq_conv_geom &g, int F, int64_t rows, const WgradCfg &c) {
-    return dense_shape(g, F) ? gemm_parts_splits(rows, g.C, F) : wgrad_splits(rows, c.n_kt * c.n_nt);
+    return dense_shape(g, F) || wgrad_parts(g, F) ? gemm_parts_splits(rows, g.kh * g.kw * g.C, F) : wgrad_splits(rows, c.n_kt * c.n_nt);
 }
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1664,6 +1668,8 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
     }
     if (nz == 1 && conv_thin_fwd_ok(*g, F)) return conv_thin_fwd(xq, qw, qb, y, *g, F, act, s);
     if (nz == 1 && aligned16(xq) && conv_patch_ok(0, *g, F)) return conv_patch_launch(0, xq, nullptr, qw, qb, y, *g, F, act, s);
+    // (300 x 11 x 11, 3 x 3, 40 -> 40: 22 -> 15 us; 1024 x 13 x 13, 37 -> 37: 135 -> 51 us against the implicit GEMM below)
+    if (nz == 1 && conv_parts_shape(*g, F)) return conv_parts_fwd(xq, qw, qb, y, *g, F, act, s);
     const bool vec = g->C % 4 == 0 && aligned16(xq) && (int64_t)g->B * g->H * g->W * g->C * 4 < (1ll << 31);
     if (F <= 32) {
         const dim3 grid((unsigned)persistent_grid((rows + 127) / 128, vec ? 3 : 8), 1, (unsigned)nz);
@@ -1790,6 +1796,8 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
 #undef HGQ_DG
         } else if (aligned16(dy) && (!mask || aligned16(mask)) && conv_patch_ok(1, *g, F)) {
             if ((rc = conv_patch_launch(1, dy, mask, qw, nullptr, dxq, *g, F, act, s))) return rc;
+        } else if (g->sy == 1 && g->sx == 1 && conv_parts_shape(*g, F)) {  // 300 x 11 x 11, 3 x 3, 40 -> 40: 50 -> 27 us
+            if ((rc = conv_parts_dgrad(dy, act == HGQ_ACT_RELU ? mask : nullptr, qw, dxq, *g, F, s))) return rc;
         } else {
             const bool vec = F % 4 == 0 && aligned16(dy) && (!mask || aligned16(mask)) && rows * F * 4 < (1ll << 31);
             if (g->C <= 32) {
@@ -1816,6 +1824,10 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
         }
         const WgradCfg c = wgrad_cfg(K, F);
         int64_t splits = wgrad_slices(*g, F, rows, c);
+        if (!patch_shape && wgrad_parts(*g, F)) {
+            if ((rc = conv_parts_wgrad(xq, dy, act == HGQ_ACT_RELU ? mask : nullptr, workspace, *g, F, splits, s))) return rc;
+            return reduce ? reduce_parts(workspace, (int)splits, M, dqw, KF, dqb, (int64_t)F, nullptr, 0, s) : HGQ_OK;
+        }
         if (patch_shape) {
             if (splits > patch_slices) splits = patch_slices;
             if (splits < patch_slices && !reduce && (rc = fill_f32(workspace + splits * M, 0.f, (patch_slices - splits) * M, s))) return rc;

@@ -5,6 +5,10 @@
 //   data gradient  dX[m, k] = sum_n dZ[m, n] W[k, n]              dZ = dY where Y > 0 (ReLU), else dY
 //   weight grad.   dW[k, n] = sum_m X[m, k] dZ[m, n],  db[n] = sum_m dZ[m, n]      (split along m, one slice per split)
 //
+// and, with the gathered operand read through the image's geometry (CONV), the same three products of a convolution: X[m, k] is
+// the input value tap k = (ky, kx, c) of pixel m meets, the data gradient gathers dZ around an input pixel (unit stride).
+// Depths of a tap are padded to a multiple of four, so a thread's four consecutive steps are one 128-bit load.
+//
 // An operand element is split into its parts ONCE per tile, on its way into LDS, where each part has a plane of its own with
 // eight consecutive contraction steps of a row in 16 bytes: an operand of the matrix instruction is one 128-bit LDS read.
 // (The implicit-GEMM kernels these replaced read their operands as single fp32 words - 32 LDS reads per instruction - and
@@ -45,6 +49,9 @@ struct GpArgs {
     int per_xcd;            // workgroups per XCD: consecutive ones (same rows, next columns) share an L2
     int act;
     hgq_stack_quant oq;     // FWD: quantizer of the output's columns (oq.i NULL: none)
+    hgq_conv_geom cg;       // CONV
+    int depth, dp;          // CONV, FWD / DGRAD: values of a tap (C / F), padded to a multiple of four; kc = taps * dp
+    int64_t a_bytes;        // CONV: size of the gathered tensor
 };
 
 // Staging of one operand tile of S rows (output index) x BK contraction steps by 256 threads.
@@ -83,6 +90,84 @@ struct GpTile {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) m[4 * p + j] = u[j];
                 }
+            }
+        }
+    }
+    // ---- gathered operands of a convolution
+    // rows of this thread (KMAJOR false): place of the window's first tap, ~0 in `px` for rows past the end
+    int px[KMAJOR ? 1 : NP], yx[KMAJOR ? 1 : NP];
+    template <bool TRANSPOSED>
+    __device__ __forceinline__ void locate(const hgq_conv_geom &g, int64_t row0, int64_t rows) {
+        const int w = TRANSPOSED ? g.W : g.OW, per = TRANSPOSED ? g.H * g.W : g.OH * g.OW;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const int64_t m = row0 + (int)threadIdx.x / QPR + p * RPP;
+            const int b = (int)(m / per), rem = (int)(m - (int64_t)b * per), y = rem / w, x = rem - y * w;
+            px[p] = m < rows ? b * (TRANSPOSED ? g.OH * g.OW : g.H * g.W) : -1;
+            const int y0 = TRANSPOSED ? y + g.py : y * g.sy - g.py, x0 = TRANSPOSED ? x + g.px : x * g.sx - g.px;
+            yx[p] = (int)(((uint32_t)y0 << 16) | ((uint32_t)x0 & 0xffffu));
+        }
+    }
+    // four consecutive steps (tap, d0 ..) of this thread's rows from the image `base`
+    template <bool TRANSPOSED>
+    __device__ __forceinline__ void gather(__amdgpu_buffer_rsrc_t r, __amdgpu_buffer_rsrc_t rm, const hgq_conv_geom &g, int depth, int dp,
+                                           const FastDiv &by_dp, const FastDiv &by_kw, int step0, int kc) {
+        const int k = step0 + 4 * ((int)threadIdx.x % QPR), tap = (int)by_dp.div((uint32_t)k), d0 = k - tap * dp;
+        const int ky = (int)by_kw.div((uint32_t)tap), kx = tap - ky * g.kw;
+        const int h = TRANSPOSED ? g.OH : g.H, w = TRANSPOSED ? g.OW : g.W;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const int y0 = yx[p] >> 16, x0 = (int)(int16_t)(yx[p] & 0xffff);
+            const int y = TRANSPOSED ? y0 - ky * g.dly : y0 + ky * g.dly, x = TRANSPOSED ? x0 - kx * g.dlx : x0 + kx * g.dlx;
+            const bool ok = px[p] >= 0 && k < kc && (unsigned)y < (unsigned)h && (unsigned)x < (unsigned)w;
+            const uint32_t off = ok ? (uint32_t)((px[p] + y * w + x) * depth + d0) * 4u : BUF_OOB;
+            const f32x4_t t = gp_ld4(r, off, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[4 * p + j] = depth == dp || d0 + j < depth ? t[j] : 0.f;
+            if (MASKED) {
+                const f32x4_t u = gp_ld4(rm, off, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) m[4 * p + j] = u[j];
+            }
+        }
+    }
+    // DGRAD: kernel entries w[tap][c][f], rows c of this tile from c0, four consecutive f
+    __device__ __forceinline__ void kernel_rows(__amdgpu_buffer_rsrc_t r, int c0, int C, int F, int dp, const FastDiv &by_dp, int step0, int kc) {
+        const int k = step0 + 4 * ((int)threadIdx.x % QPR), tap = (int)by_dp.div((uint32_t)k), f0 = k - tap * dp;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const int c = c0 + (int)threadIdx.x / QPR + p * RPP;
+            const f32x4_t t = gp_ld4(r, c < C && k < kc ? (uint32_t)((tap * C + c) * F + f0) * 4u : BUF_OOB, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[4 * p + j] = f0 + j < F ? t[j] : 0.f;
+        }
+    }
+    // FWD: kernel entries w[tap][c][n], column n of this tile, consecutive steps
+    __device__ __forceinline__ void kernel_cols(__amdgpu_buffer_rsrc_t r, int n0, int C, int F, int dp, const FastDiv &by_dp, int step0, int kc) {
+        const int n = n0 + (int)threadIdx.x % S, k0 = step0 + ((int)threadIdx.x / S) * N;
+#pragma unroll
+        for (int q = 0; q < N / 4; ++q) {
+            const int k = k0 + 4 * q, tap = (int)by_dp.div((uint32_t)k), c0 = k - tap * dp;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[4 * q + j] = gp_ld1(r, n < F && k < kc && c0 + j < C ? (uint32_t)((tap * C + c0 + j) * F + n) * 4u : BUF_OOB, 0);
+        }
+    }
+    // WGRAD: this thread's kernel entry (output row) against consecutive pixels from m0 on
+    __device__ __forceinline__ void pixels(__amdgpu_buffer_rsrc_t r, const hgq_conv_geom &g, int k, int K, int64_t m0, int64_t m_end) {
+        const int tap = k / g.C, c = k - tap * g.C, ky = tap / g.kw, kx = tap - ky * g.kw;
+        const int dy = ky * g.dly - g.py, dx = kx * g.dlx - g.px;
+        // the pixels are the same for a whole wavefront (S >= 64 columns)
+        const int mm = (int)m0 + __builtin_amdgcn_readfirstlane((int)threadIdx.x / S) * N, per = g.OH * g.OW;
+        int b = mm / per, oy = (mm - b * per) / g.OW, ox = mm - b * per - oy * g.OW;
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            const int y = oy * g.sy + dy, x = ox * g.sx + dx;
+            const bool ok = k < K && mm + e < (int)m_end && (unsigned)y < (unsigned)g.H && (unsigned)x < (unsigned)g.W;
+            v[e] = gp_ld1(r, ok ? (uint32_t)(((b * g.H + y) * g.W + x) * g.C + c) * 4u : BUF_OOB, 0);
+            if (++ox == g.OW) {
+                ox = 0;
+                if (++oy == g.OH) oy = 0, ++b;
             }
         }
     }
@@ -145,7 +230,7 @@ struct GpTile {
     }
 };
 
-template <int OP, int BM, int BN, int BK>
+template <int OP, int BM, int BN, int BK, bool CONV>
 __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
     constexpr bool A_KMAJOR = OP == GP_WGRAD, B_KMAJOR = OP != GP_DGRAD;
     constexpr int WN = BN >= 64 ? 2 : 1, WM = 4 / WN;    // wavefronts along the rows / columns of the tile
@@ -175,8 +260,23 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
     TA ta;
     TB tb;
     float bsum = 0.f;
+    const FastDiv by_dp((uint32_t)(CONV ? g.dp : 1)), by_kw((uint32_t)(CONV ? g.cg.kw : 1));
+    const int64_t w_bytes = CONV ? (int64_t)g.cg.kh * g.cg.kw * g.cg.C * (OP == GP_DGRAD ? g.depth : g.no) * 4 : 0;
+    const __amdgpu_buffer_rsrc_t rs_a = buf_rsrc(g.a, CONV ? g.a_bytes : 0), rs_w = buf_rsrc(g.b, w_bytes),
+                                 rs_m = buf_rsrc(CONV && relu ? g.mask : g.a, CONV && relu ? g.a_bytes : 0);
+    if (CONV && OP != GP_WGRAD) ta.template locate<OP == GP_DGRAD>(g.cg, r0, g.rows);
     auto fetch = [&](int st) {
-        if (OP == GP_WGRAD) {
+        if (CONV && OP == GP_FWD) {
+            ta.template gather<false>(rs_a, rs_m, g.cg, g.depth, g.dp, by_dp, by_kw, st * BK, g.kc);
+            tb.kernel_cols(rs_w, n0, g.depth, g.no, g.dp, by_dp, st * BK, g.kc);
+        } else if (CONV && OP == GP_DGRAD) {
+            ta.template gather<true>(rs_a, rs_m, g.cg, g.depth, g.dp, by_dp, by_kw, st * BK, g.kc);
+            tb.kernel_rows(rs_w, n0, g.no, g.depth, g.dp, by_dp, st * BK, g.kc);
+        } else if (CONV) {
+            const int64_t m0 = c_begin + (int64_t)st * BK, left = c_end - m0;
+            ta.pixels(rs_a, g.cg, (int)r0 + tid % BM, g.mo, m0, c_end);
+            tb.fetch(g.b + m0 * g.no + n0, relu ? g.mask + m0 * g.no + n0 : nullptr, (left * g.no - n0) * 4, g.no, g.no - n0, 0);
+        } else if (OP == GP_WGRAD) {
             const int64_t m0 = c_begin + (int64_t)st * BK;
             const int64_t left = c_end - m0;
             ta.fetch(g.a + m0 * g.mo + r0, nullptr, (left * g.mo - r0) * 4, g.mo, g.mo - (int)r0, 0);
@@ -195,7 +295,7 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
     if (n_steps > 0) fetch(0);
     for (int st = 0; st < n_steps; ++st) {
         const int left = (int)min((int64_t)BK, c_end - c_begin - (int64_t)st * BK);
-        ta.clip(left), tb.clip(left);
+        if (!CONV) ta.clip(left), tb.clip(left);
         ta.mask(relu), tb.mask(relu);
         if (OP == GP_WGRAD) {
             if (mt == 0) {
@@ -284,13 +384,33 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) < INFINITY);
     if (__any(bad)) {
+        // CONV: value of the gathered tensor that pixel m and depth d of tap `tap` meet
+        auto tap_at = [&](int64_t m, int tap, int d) -> float {
+            const hgq_conv_geom &q = g.cg;
+            const int ky = tap / q.kw, kx = tap - ky * q.kw;
+            const int per = OP == GP_DGRAD ? q.H * q.W : q.OH * q.OW, w = OP == GP_DGRAD ? q.W : q.OW;
+            const int b = (int)(m / per), rem = (int)(m - (int64_t)b * per), y = rem / w, x = rem - y * w;
+            const int sy = OP == GP_DGRAD ? y + q.py - ky * q.dly : y * q.sy - q.py + ky * q.dly;
+            const int sx = OP == GP_DGRAD ? x + q.px - kx * q.dlx : x * q.sx - q.px + kx * q.dlx;
+            const int sh = OP == GP_DGRAD ? q.OH : q.H, sw = OP == GP_DGRAD ? q.OW : q.W, depth = OP == GP_WGRAD ? q.C : g.depth;
+            if ((unsigned)sy >= (unsigned)sh || (unsigned)sx >= (unsigned)sw) return 0.f;
+            const int64_t e = (((int64_t)b * sh + sy) * sw + sx) * depth + d;
+            return OP == GP_DGRAD && relu && !(g.mask[e] > 0.f) ? 0.f : g.a[e];
+        };
         auto a_at = [&](int64_t i, int64_t c) -> float {  // output row i of the tile's matrix, contraction step c
             if (c >= c_end || i >= (OP == GP_WGRAD ? (int64_t)g.mo : g.rows)) return 0.f;
+            if (CONV && OP == GP_WGRAD) return tap_at(c, (int)i / g.cg.C, (int)i % g.cg.C);
+            if (CONV) return (int)c % g.dp < g.depth ? tap_at(i, (int)c / g.dp, (int)c % g.dp) : 0.f;
             const int64_t e = A_KMAJOR ? c * g.mo + i : i * g.kc + c;
             return OP == GP_DGRAD && relu && !(g.mask[e] > 0.f) ? 0.f : g.a[e];
         };
         auto b_at = [&](int64_t j, int64_t c) -> float {
             if (c >= c_end || j >= g.no) return 0.f;
+            if (CONV && OP != GP_WGRAD) {
+                const int tap = (int)c / g.dp, d = (int)c - tap * g.dp;
+                if (d >= g.depth) return 0.f;
+                return OP == GP_FWD ? g.b[((int64_t)tap * g.depth + d) * g.no + j] : g.b[((int64_t)tap * g.no + j) * g.depth + d];
+            }
             const int64_t e = B_KMAJOR ? c * g.no + j : j * g.kc + c;
             return OP == GP_WGRAD && relu && !(g.mask[e] > 0.f) ? 0.f : g.b[e];
         };
@@ -348,13 +468,13 @@ __global__ __launch_bounds__(256, 2) void gemm_parts_kernel(const GpArgs g) {
     }
 }
 
-template <int OP, int BM, int BN, int BK>
+template <int OP, int BM, int BN, int BK, bool CONV = false>
 static void gp_launch(GpArgs g, int splits, hipStream_t s) {
     g.ntm = (int)(((OP == GP_WGRAD ? (int64_t)g.mo : g.rows) + BM - 1) / BM);
     g.ntn = (g.no + BN - 1) / BN;
     g.total = g.ntm * g.ntn * splits;
     g.per_xcd = (g.total + 7) / 8;
-    hipLaunchKernelGGL((gemm_parts_kernel<OP, BM, BN, BK>), dim3((unsigned)g.per_xcd * 8u), dim3(256), 0, s, g);
+    hipLaunchKernelGGL((gemm_parts_kernel<OP, BM, BN, BK, CONV>), dim3((unsigned)g.per_xcd * 8u), dim3(256), 0, s, g);
 }
 
 // Tile of a product with `m` x `n` outputs.  128 x 128 tiles split and stage each operand value half as often, but a launch
@@ -403,6 +523,44 @@ int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *
     if (N <= 32) gp_launch<GP_WGRAD, 128, 32, 32>(g, (int)splits, s);
     else gp_launch<GP_WGRAD, 64, 64, 64>(g, (int)splits, s);
     return check_launch("gemm_parts(weight gradient)");
+}
+
+// ---- convolutions.  Pixel indices and places in a window are 32- and 16-bit numbers, tensors below 2 GiB.
+bool conv_parts_shape(const hgq_conv_geom &g, int F) {
+    const int lim = 16384;
+    return hgq_dense_use_bf16_parts(-1) != 0 && g.H <= lim && g.W <= lim && g.OH <= lim && g.OW <= lim && g.py <= lim / 2 && g.px <= lim / 2 &&
+           (int64_t)g.OH * g.sy <= lim && (int64_t)g.OW * g.sx <= lim && (int64_t)g.kh * g.dly <= lim && (int64_t)g.kw * g.dlx <= lim &&
+           (int64_t)g.kh * g.kw * (g.C + 3) < (1 << 20) && (int64_t)g.kh * g.kw * (F + 3) < (1 << 20) && F <= (1 << 16) &&
+           (int64_t)g.kh * g.kw * g.C * F * 4 < (1ll << 31) && (int64_t)g.B * g.H * g.W * g.C * 4 < (1ll << 31) &&
+           (int64_t)g.B * g.OH * g.OW * F * 4 < (1ll << 31);
+}
+
+int conv_parts_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &cg, int F, int act, hipStream_t s) {
+    GpArgs g = {};
+    g.a = x, g.b = w, g.bias = bias, g.out = y, g.rows = (int64_t)cg.B * cg.OH * cg.OW, g.no = F, g.act = act, g.cg = cg;
+    g.depth = cg.C, g.dp = (cg.C + 3) & ~3, g.kc = cg.kh * cg.kw * g.dp, g.a_bytes = (int64_t)cg.B * cg.H * cg.W * cg.C * 4;
+    if (F <= 32) gp_launch<GP_FWD, 128, 32, 32, true>(g, 1, s);
+    else gp_launch<GP_FWD, 64, 64, 64, true>(g, 1, s);
+    return check_launch("hgq_conv2d_fwd(parts)");
+}
+
+int conv_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, const hgq_conv_geom &cg, int F, hipStream_t s) {
+    GpArgs g = {};
+    g.a = dy, g.b = w, g.mask = mask, g.out = dx, g.rows = (int64_t)cg.B * cg.H * cg.W, g.no = cg.C, g.cg = cg;
+    g.depth = F, g.dp = (F + 3) & ~3, g.kc = cg.kh * cg.kw * g.dp, g.a_bytes = (int64_t)cg.B * cg.OH * cg.OW * F * 4;
+    if (cg.C <= 32) gp_launch<GP_DGRAD, 128, 32, 32, true>(g, 1, s);
+    else gp_launch<GP_DGRAD, 64, 64, 64, true>(g, 1, s);
+    return check_launch("hgq_conv2d_bwd(data, parts)");
+}
+
+int conv_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, const hgq_conv_geom &cg, int F, int64_t splits, hipStream_t s) {
+    GpArgs g = {};
+    g.a = x, g.b = dy, g.mask = mask, g.out = part, g.rows = (int64_t)cg.B * cg.OH * cg.OW, g.mo = cg.kh * cg.kw * cg.C, g.no = F, g.cg = cg;
+    g.a_bytes = (int64_t)cg.B * cg.H * cg.W * cg.C * 4;
+    g.chunk = ((g.rows + splits - 1) / splits + 63) / 64 * 64;
+    if (F <= 32) gp_launch<GP_WGRAD, 128, 32, 32, true>(g, (int)splits, s);
+    else gp_launch<GP_WGRAD, 64, 64, 64, true>(g, (int)splits, s);
+    return check_launch("hgq_conv2d_bwd(weights, parts)");
 }
 
 }  // namespace hgq

@@ -61,6 +61,12 @@ int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *
 int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits,
                      hipStream_t s);
 
+// Convolutions of any geometry on the same kernels (the data gradient: unit stride); `splits`: gemm_parts_splits(pixels, K, F).
+bool conv_parts_shape(const hgq_conv_geom &g, int F);
+int conv_parts_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);
+int conv_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, const hgq_conv_geom &g, int F, hipStream_t s);
+int conv_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, const hgq_conv_geom &g, int F, int64_t splits, hipStream_t s);
+
 // Convolutions over few input values per pixel (hgq_conv_thin.hip): which shapes, the slices the backward pass leaves
 // ([K F + F] each), forward, and data + weight + bias gradient in one pass.
 bool conv_thin_fwd_ok(const hgq_conv_geom &g, int F);
