@@ -190,7 +190,7 @@ class StackQuant(ctypes.Structure):
 class StackLayer(ctypes.Structure):
     """``hgq_stack_layer`` of include/hgq_hip.h."""
 
-    _fields_ = [('w', c_void_p), ('bias', c_void_p), ('kq', StackQuant), ('bq', StackQuant), ('iq', StackQuant),
+    _fields_ = [('w', c_void_p), ('bias', c_void_p), ('kq', StackQuant), ('bq', StackQuant), ('iq', StackQuant), ('oq', StackQuant),
                 ('K', c_int), ('N', c_int), ('act', c_int)]
 
 

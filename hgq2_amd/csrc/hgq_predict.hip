@@ -73,7 +73,7 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
             }
         }
         if (h.bias && tid < h.N) w[Kp * Np + tid] = stack_quantize(h.bias[tid], stack_entry(h.bq, stack_index(h.bq, tid, h.N)), h.bq.mode);
-        if (h.iq.i && tid >= 64 && tid < 64 + h.K) {
+        if (h.iq.i && h.iq.size <= h.K && tid >= 64 && tid < 64 + h.K) {
             const int c = tid - 64;
             const KIF p = stack_entry(h.iq, h.iq.size == 1 ? 0 : c);
             qt[l * 192 + c] = p.k, qt[l * 192 + 64 + c] = p.i, qt[l * 192 + 128 + c] = p.f;
@@ -90,17 +90,25 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
         {
             // the input tile: rows are contiguous; zeros past the last one (their results are not stored)
             const __amdgpu_buffer_rsrc_t rs = buf_rsrc(x + r0 * K0, (int64_t)live * K0 * 4);
-            const bool quant = d.l[0].iq.i != nullptr;
+            const hgq_stack_quant &iq = d.l[0].iq;
+            const bool quant = iq.i != nullptr, table = quant && iq.size > K0;  // (a table of several rows is read per element)
+            const int t0 = table ? (int)(r0 * K0 % iq.size) : 0;
             for (int e0 = tid; e0 < CHAIN_BM * K0; e0 += 4 * CHAIN_NT) {
                 float v[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) v[u] = buf_ld1(rs, e0 + u * CHAIN_NT < CHAIN_BM * K0 ? (uint32_t)(e0 + u * CHAIN_NT) * 4u : BUF_OOB);
+                KIF p[4];
+                if (table) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) p[u] = stack_entry(iq, (t0 + e0 + u * CHAIN_NT) % iq.size);
+                }
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     const int e = e0 + u * CHAIN_NT;
                     if (e < CHAIN_BM * K0) {
                         const int row = (int)by_k0.div((uint32_t)e), c = e - row * K0;
-                        tiles[row * CHAIN_LD + c] = quant ? stack_quantize(v[u], KIF{qt[c], qt[64 + c], qt[128 + c]}, d.l[0].iq.mode) : v[u];
+                        if (!table) p[u] = KIF{qt[c], qt[64 + c], qt[128 + c]};
+                        tiles[row * CHAIN_LD + c] = quant ? stack_quantize(v[u], p[u], iq.mode) : v[u];
                     }
                 }
             }
@@ -138,9 +146,20 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
         }
         __syncthreads();
         const float *out = tiles + (L & 1) * CHAIN_BM * CHAIN_LD;
-        for (int e = tid; e < live * NL; e += CHAIN_NT) {
-            const int row = (int)by_nl.div((uint32_t)e);
-            y[r0 * NL + e] = out[row * CHAIN_LD + (e - row * NL)];
+        const hgq_stack_quant &oq = d.l[L - 1].oq;
+        const int t0 = oq.i ? (int)(r0 * NL % oq.size) : 0;
+        for (int e0 = tid; e0 < live * NL; e0 += 4 * CHAIN_NT) {
+            float v[4];
+            KIF p[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = e0 + u * CHAIN_NT < live * NL ? e0 + u * CHAIN_NT : e0, row = (int)by_nl.div((uint32_t)e);
+                v[u] = out[row * CHAIN_LD + (e - row * NL)];
+                if (oq.i) p[u] = stack_entry(oq, oq.size == 1 ? 0 : (t0 + e) % oq.size);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (e0 + u * CHAIN_NT < live * NL) y[r0 * NL + e0 + u * CHAIN_NT] = oq.i ? stack_quantize(v[u], p[u], oq.mode) : v[u];
         }
         __syncthreads();  // the next input tile goes into the first buffer
     }
@@ -187,7 +206,8 @@ static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
         const hgq_stack_layer &h = layers[l];
         if (h.K < 1 || h.N < 1 || (int64_t)h.K * h.N > (1 << 26) || (l && h.K != layers[l - 1].N)) return 0;
         if (!h.w || !quant_ok(h.kq, (int64_t)h.K * h.N) || (h.bias && !quant_ok(h.bq, h.N))) return 0;
-        if (h.iq.i && (!quant_ok(h.iq, h.K) || h.iq.inner != 1 || (h.iq.size != 1 && h.iq.size != h.K))) return 0;
+        if (h.iq.i && (!quant_ok(h.iq, l ? h.K : rows * h.K) || h.iq.inner != 1 || (h.iq.size != 1 && (l ? h.iq.size != h.K : h.iq.size % h.K)))) return 0;
+        if (h.oq.i && (l + 1 < n || !quant_ok(h.oq, rows * h.N) || h.oq.inner != 1 || (h.oq.size != 1 && h.oq.size % h.N))) return 0;
         chain = chain && h.K <= 64 && h.N <= 64;
         wide = wide && gemm_parts_shape(rows, h.K, h.N);
     }
@@ -201,9 +221,11 @@ static int64_t image_floats(const hgq_stack_layer *layers, int n) {
     for (int l = 0; l < n; ++l) at += ((int64_t)layers[l].K * layers[l].N + 3) / 4 * 4 + (layers[l].N + 3) / 4 * 4;
     return at;
 }
-// widest tensor that goes into buffer `which` (0: inputs of even layers, 1: of odd layers)
+// an output quantizer the last product's epilogue does not apply (it takes one entry or one per column)
+static bool table_out(const hgq_stack_layer &h) { return h.oq.i && h.oq.size > h.N; }
+// widest tensor that goes into buffer `which` (0: inputs of even layers, 1: of odd layers, and a last output to be quantized)
 static int64_t buffer_floats(const hgq_stack_layer *layers, int n, int64_t rows, int which) {
-    int64_t w = 0;
+    int64_t w = table_out(layers[n - 1]) && (n & 1) == which ? layers[n - 1].N : 0;
     for (int l = which; l < n; l += 2)
         if ((l || layers[0].iq.i) && layers[l].K > w) w = layers[l].K;
     return (w * rows + 3) / 4 * 4;
@@ -262,9 +284,11 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
     }
     for (int l = 0; l < n_layers; ++l) {
         const hgq_stack_layer &h = layers[l];
-        float *out = l + 1 == n_layers ? y : buf[(l + 1) & 1];
-        const hgq_stack_quant *oq = l + 1 < n_layers && layers[l + 1].iq.i ? &layers[l + 1].iq : nullptr;
+        const bool last = l + 1 == n_layers, later = last && table_out(h);
+        float *out = last && !later ? y : buf[(l + 1) & 1];
+        const hgq_stack_quant *oq = last ? (h.oq.i && !later ? &h.oq : nullptr) : layers[l + 1].iq.i ? &layers[l + 1].iq : nullptr;
         if ((rc = gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq))) return rc;
+        if (later) return hgq_quantize_fwd(out, h.oq.k, h.oq.i, h.oq.fb, y, nullptr, nullptr, rows * h.N, h.oq.size, 1, h.oq.mode, stream);
         cur = out;
     }
     return HGQ_OK;

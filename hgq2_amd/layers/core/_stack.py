@@ -11,7 +11,6 @@ from ... import _lib, ops
 from ...quantizer.internal import FixedPointQuantizerKBI, FixedPointQuantizerKIF
 from ...quantizer.internal.base import bw_layout
 from ...quantizer.quantizer import Quantizer
-from .dense import QDense
 
 _ACTS = {None: _lib.ACT_NONE, 'linear': _lib.ACT_NONE, 'relu': _lib.ACT_RELU}
 
@@ -56,31 +55,44 @@ def _describe(q, shape, device, out) -> bool:
     return True
 
 
-def _layer(layer, rows, k_in, device, out) -> bool:
-    """Fill ``out`` for one layer; False where its call is more than quantize, contract, add, activate."""
-    if type(layer) is not QDense or not layer.built or layer._enable_oq or layer._act_name not in _ACTS or 'call' in layer.__dict__:
+def _contraction(layer, K, N, device, out) -> bool:
+    """Fill ``out`` with the kernel, bias and activation of a layer that contracts ``[rows, K]`` with its variables' ``[K, N]``
+    view; False where its call does more than quantize, contract, add, activate."""
+    if not layer.built or layer._act_name not in _ACTS or 'call' in layer.__dict__:
         return False
     w, b = layer._parameters.get('_kernel'), layer._parameters.get('bias')
-    if w is None or layer._kq is None or w.dim() != 2 or w.shape[0] != k_in or w.dtype is not torch.float32 or w.device != device or not w.is_contiguous():
+    if w is None or layer._kq is None or w.numel() != K * N or w.dtype is not torch.float32 or w.device != device or not w.is_contiguous():
         return False
     if not _describe(layer._kq, w.shape, device, out.kq):
         return False
-    out.w, out.K, out.N, out.act = w.data_ptr(), k_in, w.shape[1], _ACTS[layer._act_name]
+    out.w, out.K, out.N, out.act = w.data_ptr(), K, N, _ACTS[layer._act_name]
     if b is not None:
-        if layer._bq is None or b.dtype is not torch.float32 or b.device != device or not b.is_contiguous() or b.numel() != out.N:
+        if layer._bq is None or b.dtype is not torch.float32 or b.device != device or not b.is_contiguous() or b.numel() != N:
             return False
         if not _describe(layer._bq, b.shape, device, out.bq):
             return False
         out.bias = b.data_ptr()
-    if layer._enable_iq:
-        if not _describe(layer._iq, (rows, k_in), device, out.iq):
-            return False
-        size, inner = out.iq.size, out.iq.inner
-        if size == 1:
-            out.iq.inner = 1
-        elif size != k_in or inner != 1:
-            return False
     return True
+
+
+def _rows_quantizer(q, shape, width, device, out, rows) -> bool:
+    """Fill ``out`` for a quantizer of the contraction's input or output: one entry, or a table of ``rows`` (None: any number
+    of) rows of ``width`` columns."""
+    if not _describe(q, shape, device, out):
+        return False
+    if out.size == 1:
+        out.inner = 1
+        return True
+    return out.inner == 1 and (out.size % width == 0 if rows is None else out.size == rows * width)
+
+
+def _layer(layer, rows, k_in, device, out, first) -> bool:
+    """Fill ``out`` for one QDense layer of a run."""
+    from .dense import QDense
+
+    if type(layer) is not QDense or not layer.built or layer._enable_oq or not _contraction(layer, k_in, layer.units, device, out):
+        return False
+    return not layer._enable_iq or _rows_quantizer(layer._iq, (rows, k_in), k_in, device, out.iq, None if first else 1)
 
 
 def _ordinary_call() -> bool:
@@ -90,24 +102,47 @@ def _ordinary_call() -> bool:
                 or torch.autograd.forward_ad._current_level >= 0)
 
 
+def _plain_input(x) -> bool:
+    return (type(x) is torch.Tensor and x.is_cuda and x.dtype is torch.float32 and 0 < x.numel() < 2**31
+            and x.device.index == torch.cuda.current_device() and _ordinary_call())
+
+
+def predict_contraction(layer, x, K, N, out_shape):
+    """Output of a contraction layer's whole call - input, kernel, bias and output quantizer, contraction, activation - outside
+    training, tracing and gradients as one library call, or ``None``.  ``x`` [..., K] and the output are read as rows."""
+    if not _plain_input(x) or x.shape[0] * K > x.numel():
+        return None
+    rows, device = x.numel() // K, x.device
+    descs = (_lib.StackLayer * 1)()
+    if not _contraction(layer, K, N, device, descs[0]):
+        return None
+    if layer._enable_iq and not _rows_quantizer(layer._iq, x.shape, K, device, descs[0].iq, None):
+        return None
+    if layer._enable_oq and not _rows_quantizer(layer._oq, out_shape, N, device, descs[0].oq, None):
+        return None
+    y = ops.dense_stack_predict(x, descs, 1, rows, N)
+    if y is None:
+        return None
+    layer._deferred, layer._oq_applied_in_call = None, True
+    return y.view(out_shape)
+
+
 def predict_run(layers, first, x):
     """``(output, index behind the last layer taken)`` for the longest run of layers from ``first`` on that one library call
     covers, or ``None``."""
-    if type(x) is not torch.Tensor or not x.is_cuda or x.dtype is not torch.float32 or x.dim() != 2 or not x.numel() or not _ordinary_call():
+    if x.dim() != 2 or not _plain_input(x):
         return None
     rows, width = x.shape
     descs = (_lib.StackLayer * _lib.STACK_MAX_LAYERS)()
     n, device = 0, x.device
-    if rows > 2**30 or device.index != torch.cuda.current_device():
-        return None
     while n < _lib.STACK_MAX_LAYERS and first + n < len(layers):
-        if not _layer(layers[first + n], rows, width, device, descs[n]):
+        if not _layer(layers[first + n], rows, width, device, descs[n], n == 0):
             break
         width = descs[n].N
         n += 1
     if n == 0:
         return None
-    y = ops.dense_stack_predict(x, descs, n, width)
+    y = ops.dense_stack_predict(x, descs, n, rows, width)
     if y is None:
         return None
     for layer in layers[first:first + n]:

@@ -10,6 +10,7 @@ from ...core import get_initializer
 from ...quantizer import Quantizer
 from ...quantizer.config import QuantizerConfig
 from ._contraction import dense_contraction, dense_ebops_term, get_activation
+from ._stack import predict_contraction
 from .base import QLayerBaseSingleInput, mean_bits, scale_ebops
 
 
@@ -69,6 +70,10 @@ class QDense(QLayerBaseSingleInput):
         return tuple(input_shape[:-1]) + (self.units,)
 
     def call(self, inputs, training=None):
+        if training is False and type(self) is QDense and not torch.is_grad_enabled():
+            y = predict_contraction(self, inputs, inputs.shape[-1], self.units, tuple(inputs.shape[:-1]) + (self.units,))
+            if y is not None:
+                return y
         iq = self.iq if self.enable_iq else None
         oq = self.oq if (self.enable_oq and not self.__output_quantizer_handled__) else None
         y, act_done, self._deferred, self._oq_applied_in_call = dense_contraction(

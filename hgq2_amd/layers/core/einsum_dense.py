@@ -18,6 +18,7 @@ from ...core import get_initializer
 from ...quantizer import Quantizer
 from ...quantizer.config import QuantizerConfig
 from ._contraction import dense_contraction, dense_contraction_mean, dense_ebops_term, get_activation
+from ._stack import predict_contraction
 from .base import QLayerBaseSingleInput, mean_bits, scale_ebops
 
 
@@ -261,6 +262,11 @@ class QEinsumDense(QLayerBaseSingleInput):
         return y if mean_done else then(y)
 
     def call(self, inputs, training=None, then=None):
+        if (training is False and then is None and type(self) is QEinsumDense and not torch.is_grad_enabled() and self._gemm is not None
+                and (self.bias is None or self._bias_in_gemm) and not self.__output_quantizer_handled__):
+            y = predict_contraction(self, inputs, self._K, self._N, (inputs.shape[0],) + tuple(self.full_output_shape[1:]))
+            if y is not None:
+                return y
         qkernel = self.kq(self._kernel, training=training)
         qbias = self.bq(self.bias, training=training) if self.bias is not None else None
         if then is not None:

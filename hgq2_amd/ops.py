@@ -2603,11 +2603,10 @@ def matmul_bias_act(x2d: Tensor, qw: Tensor, qb, act: int = 0) -> Tensor:
     return y.view(rows, N)
 
 
-def dense_stack_predict(x, descs, n: int, n_out: int):
+def dense_stack_predict(x, descs, n: int, rows: int, n_out: int):
     """Output ``[rows, n_out]`` of a stack of dense layers described by the first ``n`` entries of ``descs``
     (``_lib.StackLayer``) without gradients, or ``None`` where the library does not cover it."""
     lib = _lib.load()
-    rows = x.shape[0]
     floats = lib.hgq_dense_stack_workspace(descs, n, rows)
     if floats < 0:
         return None

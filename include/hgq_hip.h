@@ -208,8 +208,10 @@ int hgq_quantize_bwd_multi(const hgq_quant_grad_item *items, int count, void *st
 /*
  * Inference of a stack of QDense layers (the composition of QDense.call with training=False,
  * src/hgq/layers/core/dense.py:72-79): y [rows, N_last] from x [rows, K_first].  Every quantizer comes as its raw variables;
- * element e of the quantized tensor uses entry (e / inner) % size of them.  Input quantizers: one entry, or one per column
- * (inner 1); iq.i == NULL: none.  bias == NULL: none.  act: HGQ_ACT_*.  A layer's K is the previous one's N.
+ * element e of the quantized tensor uses entry (e / inner) % size of them (inner 1 for inputs and outputs).  Input
+ * quantizers: one entry, or one per column; the first layer's may be a table of any number of rows that divides the rows.
+ * iq.i == NULL: none.  oq: output quantizer, on the last layer only (i == NULL: none), one entry or a table of such rows.
+ * bias == NULL: none.  act: HGQ_ACT_*.  A layer's K is the previous one's N.
  * hgq_dense_stack_workspace: floats of scratch (16-byte aligned), 0 when none is needed, -1 when the call is not covered.
  */
 #define HGQ_STACK_MAX_LAYERS 8
@@ -220,7 +222,7 @@ typedef struct {
 } hgq_stack_quant;
 typedef struct {
     const float *w, *bias;
-    hgq_stack_quant kq, bq, iq;
+    hgq_stack_quant kq, bq, iq, oq;
     int K, N, act;
 } hgq_stack_layer;
 int64_t hgq_dense_stack_workspace(const hgq_stack_layer *layers, int n_layers, int64_t rows);

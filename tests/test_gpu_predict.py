@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 from hgq2_amd import core, ops  # noqa: E402
 from hgq2_amd.config import LayerConfigScope, QuantizerConfigScope  # noqa: E402
 from hgq2_amd.core import Sequential  # noqa: E402
-from hgq2_amd.layers import QDense  # noqa: E402
+from hgq2_amd.layers import QDense, QEinsumDense  # noqa: E402
 from hgq2_amd.layers.core import _stack  # noqa: E402
 from hgq2_amd.utils.minmax_trace import trace_minmax  # noqa: E402
 
@@ -27,7 +27,7 @@ def _net(dims, datalane='kif', over='WRAP', weights='SAT_SYM', rnd='RND', iq=Tru
 
 def _layerwise(net, x, monkeypatch):
     with monkeypatch.context() as m:
-        m.setattr(_stack, 'predict_run', lambda *a: None)
+        m.setattr(_stack, '_plain_input', lambda x: False)
         with torch.no_grad():
             return net(x)
 
@@ -135,3 +135,29 @@ def test_replays_in_a_graph():
         torch.cuda.synchronize()
         with torch.no_grad():
             assert torch.equal(y, net(x))
+
+
+# tables over positions (as many rows as positions, or one), narrow and wide widths, with and without an output quantizer
+@pytest.mark.parametrize('T,K,N,H', [(1, 5, 3, 2), (50, 48, 3, 16), (7, 64, 1, 64), (33, 70, 5, 20), (64, 96, 8, 32), (10, 17, 2, 33)])
+@pytest.mark.parametrize('oq', [True, False])
+@pytest.mark.parametrize('shared', [None, (0, 1)])
+def test_projections_over_positions(T, K, N, H, oq, shared, monkeypatch):
+    g = torch.Generator().manual_seed(T + K)
+    kw = dict(homogeneous_axis=shared, heterogeneous_axis=None) if shared else {}
+    with QuantizerConfigScope(place='all', default_q_type='kbi', overflow_mode='SAT_SYM'), \
+            QuantizerConfigScope(place='datalane', default_q_type='kif', overflow_mode='WRAP', **kw), LayerConfigScope(enable_ebops=False):
+        net = QEinsumDense('btf,fnh->btnh', output_shape=(T, N, H), bias_axes='nh', enable_oq=oq)
+    core.set_default_device('cuda')
+    x = torch.randn((37, T, K), generator=g).cuda()
+    net(x)
+    _spread(net, g)
+    trace_minmax(net, x)
+    taken, inner = [], ops.dense_stack_predict
+    monkeypatch.setattr(ops, 'dense_stack_predict', lambda *a: taken.append(a[2]) or inner(*a))
+    with torch.no_grad():
+        got = net(x)
+    want = _layerwise(net, x, monkeypatch)
+    assert taken and torch.equal(got, want)
+    with torch.no_grad():
+        assert torch.equal(net(x[:1]), _layerwise(net, x[:1], monkeypatch))
+        assert net(x[:0]).shape == (0, T, N, H)
