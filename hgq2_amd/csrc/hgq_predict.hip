@@ -7,9 +7,10 @@
 //   runs on the accumulator registers.  One event through 16-64-32-32-5 is bound by latency: four loads and one rounding
 //   per kernel entry, then a short matrix-instruction chain per layer; the call takes 75 us, most of it the host's (a launch
 //   per quantizer and contraction, sixteen in all: 512 us).
-// * Wider layers: one launch quantizes all kernels and biases into the workspace, one the input; then a tiled product per
-//   layer whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less per layer).
-//   50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and contraction: 484 us).
+// * Wider layers, or many rows: one launch quantizes all kernels and biases into the workspace, one the input; then per layer
+//   a tiled product whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less), or the
+//   streaming kernel of up to 64 x 64.  50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and
+//   contraction: 484 us).
 //
 // Arithmetic per value is that of hgq_quantize_fwd and of the layer's own contraction; the variables are quantized again on
 // every call (they may have been written in between).
@@ -201,7 +202,7 @@ static int chain_layout(const hgq_stack_layer *layers, int n, ChainDev &d) {
 // 0: refused, 1: one launch, 2: a launch per layer
 static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
     if (!layers || n < 1 || n > HGQ_STACK_MAX_LAYERS || rows < 1) return 0;
-    bool chain = true, wide = true;
+    bool chain = true, wide = true, tables = false;
     for (int l = 0; l < n; ++l) {
         const hgq_stack_layer &h = layers[l];
         if (h.K < 1 || h.N < 1 || (int64_t)h.K * h.N > (1 << 26) || (l && h.K != layers[l - 1].N)) return 0;
@@ -209,11 +210,17 @@ static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
         if (h.iq.i && (!quant_ok(h.iq, l ? h.K : rows * h.K) || h.iq.inner != 1 || (h.iq.size != 1 && (l ? h.iq.size != h.K : h.iq.size % h.K)))) return 0;
         if (h.oq.i && (l + 1 < n || !quant_ok(h.oq, rows * h.N) || h.oq.inner != 1 || (h.oq.size != 1 && h.oq.size % h.N))) return 0;
         chain = chain && h.K <= 64 && h.N <= 64;
-        wide = wide && gemm_parts_shape(rows, h.K, h.N);
+        wide = wide && gemm_parts_shape(rows, h.K < 8 ? 8 : h.K, h.N);
+        tables = tables || (h.iq.i && h.iq.size > h.K) || (h.oq.i && h.oq.size > h.N);
     }
     ChainDev d;
-    if (chain && chain_layout(layers, n, d) <= CHAIN_LDS) return 1;
-    return (wide && hgq_dense_use_bf16_parts(-1) != 0) ? 2 : 0;
+    wide = wide && hgq_dense_use_bf16_parts(-1) != 0;
+    chain = chain && chain_layout(layers, n, d) <= CHAIN_LDS;
+    // One launch where the host and the launches are what a call costs.  Many rows: the streaming kernels move them faster -
+    // an attention block of three heads on 400 000 rows, four projections with tables each way: 1293 us on this kernel, 949 us on those; four
+    // layers without tables on 65 536 rows still finish before the host does (76 us).
+    if (chain && (!wide || rows <= (tables ? 32768 : 65536))) return 1;
+    return wide ? 2 : 0;
 }
 
 static int64_t image_floats(const hgq_stack_layer *layers, int n) {
@@ -287,7 +294,10 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
         const bool last = l + 1 == n_layers, later = last && table_out(h);
         float *out = last && !later ? y : buf[(l + 1) & 1];
         const hgq_stack_quant *oq = last ? (h.oq.i && !later ? &h.oq : nullptr) : layers[l + 1].iq.i ? &layers[l + 1].iq : nullptr;
-        if ((rc = gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq))) return rc;
+        rc = !oq && h.K <= 64 && h.N <= 64
+                 ? hgq_qdense_fwd(cur, nullptr, nullptr, nullptr, 0, qw[l], qb[l], out, nullptr, rows, h.K, h.N, h.act, 0, stream)
+                 : gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq);
+        if (rc) return rc;
         if (later) return hgq_quantize_fwd(out, h.oq.k, h.oq.i, h.oq.fb, y, nullptr, nullptr, rows * h.N, h.oq.size, 1, h.oq.mode, stream);
         cur = out;
     }

@@ -42,7 +42,7 @@ def _spread(net, g):
 
 
 @pytest.mark.parametrize('dims,rows', [((16, 64, 32, 32, 5), 1), ((1, 1), 3), ((17, 33, 64, 2), 63), ((64,) * 8, 65), ((3, 5, 31, 32, 33, 16), 130),
-                                       ((30, 20), 40000), ((64,) * 9, 70), ((8, 65, 10), 1), ((100, 130, 31, 77), 257), ((256, 512, 128, 10), 1031),
+                                       ((30, 20), 40000), ((6, 33, 64, 5), 70001), ((64,) * 9, 70), ((8, 65, 10), 1), ((100, 130, 31, 77), 257), ((256, 512, 128, 10), 1031),
                                        ((65, 3, 64), 20)])
 @pytest.mark.parametrize('kw', [dict(), dict(datalane='kbi', over='SAT', weights='SAT', rnd='RND_CONV'), dict(over='SAT_SYM', rnd='TRN', bias=False),
                                 dict(homogeneous_axis=(0, 1), heterogeneous_axis=None)])
@@ -161,3 +161,5 @@ def test_projections_over_positions(T, K, N, H, oq, shared, monkeypatch):
     with torch.no_grad():
         assert torch.equal(net(x[:1]), _layerwise(net, x[:1], monkeypatch))
         assert net(x[:0]).shape == (0, T, N, H)
+        many = x.repeat(40000 // (37 * T) + 2, 1, 1)  # beyond the rows one launch takes
+        assert torch.equal(net(many), _layerwise(net, many, monkeypatch))
