@@ -344,8 +344,8 @@ __global__ __launch_bounds__(Q1D_BS) void quant_fwd_bwd_pe(const f32x4 *__restri
 // ------------------------------------------------------------------------------------------
 // Row batches of the per-column kernels: a thread has QC_U rows of its column group in flight
 // (buffer loads; rows past the end of the workgroup's chunk read as zero, which is neutral for
-// every reduction below), and a workgroup walks a contiguous chunk of rows so that a column sees
-// few workgroups - and few atomics - at the end.
+// every reduction below), and a workgroup walks a contiguous chunk of rows (forward) or every so many
+// batches (backward) so that a column sees few workgroups - and few atomics - at the end.
 #define QC_U 8
 #define QC_BWD_U 4
 template <int VEC>
@@ -487,7 +487,7 @@ template <int RM, int OM, int VEC>
 __global__ __launch_bounds__(256) void quant_bwd_cols(const float *__restrict__ dy, const float *__restrict__ x,
                                                       const void *__restrict__ k, const float *__restrict__ i,
                                                       const float *__restrict__ fb, float *__restrict__ dx, float *di,
-                                                      float *dfb, int64_t rows, int64_t M, int TX, int64_t rows_per_wg, int mode,
+                                                      float *dfb, int64_t rows, int64_t M, int TX, int mode,
                                                       float *part) {
     const Mode m(mode);
     const int TY = 256 / TX;
@@ -1133,9 +1133,9 @@ static int quantize_bwd_sliced_impl(const float *dy, const float *x, const void 
     const int64_t M = bw_size, rows = n / M;
     HGQ_DISPATCH_RM_OM(m.round_mode, m.overflow_mode, {
         if (vec)
-            hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 4>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, rows_per_wg, mode, workspace);
+            hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 4>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, mode, workspace);
         else
-            hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 1>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, rows_per_wg, mode, workspace);
+            hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 1>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, mode, workspace);
     });
     int rc = check_launch("hgq_quantize_bwd_sliced");
     if (rc || !reduce) return rc;
@@ -1251,9 +1251,9 @@ extern "C" int hgq_quantize_bwd(const float *dy, const float *x, const void *k, 
         cols_grid(rows, M, TY * QC_BWD_U, gx, gy, rows_per_wg);
         HGQ_DISPATCH_RM_OM(m.round_mode, m.overflow_mode, {
             if (vec)
-                hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 4>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, rows_per_wg, mode, (float *)nullptr);
+                hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 4>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, mode, (float *)nullptr);
             else
-                hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 1>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, rows_per_wg, mode, (float *)nullptr);
+                hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 1>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, mode, (float *)nullptr);
         });
         return check_launch("hgq_quantize_bwd");
     }
