@@ -12,9 +12,6 @@ from ...quantizer.internal import FixedPointQuantizerKBI, FixedPointQuantizerKIF
 from ...quantizer.internal.base import bw_layout
 from ...quantizer.quantizer import Quantizer
 
-_ACTS = {None: _lib.ACT_NONE, 'linear': _lib.ACT_NONE, 'relu': _lib.ACT_RELU}
-
-
 @functools.lru_cache(maxsize=1024)
 def _mode(round_mode, overflow_mode, training, kbi, symmetric):
     return _lib.mode_bits(round_mode, overflow_mode, training=training, kbi=kbi, round_params=True, k_u8=True, symmetric=symmetric)
@@ -58,14 +55,18 @@ def _describe(q, shape, device, out) -> bool:
 def _contraction(layer, K, N, device, out) -> bool:
     """Fill ``out`` with the kernel, bias and activation of a layer that contracts ``[rows, K]`` with its variables' ``[K, N]``
     view; False where its call does more than quantize, contract, add, activate."""
-    if not layer.built or layer._act_name not in _ACTS or 'call' in layer.__dict__:
+    if not layer.built or 'call' in layer.__dict__:
+        return False
+    # as the layers' own calls do: a ReLU by name runs inside the contraction, any other activation object behind it
+    if layer._act_name != 'relu' and layer.activation is not None:
         return False
     w, b = layer._parameters.get('_kernel'), layer._parameters.get('bias')
     if w is None or layer._kq is None or w.numel() != K * N or w.dtype is not torch.float32 or w.device != device or not w.is_contiguous():
         return False
     if not _describe(layer._kq, w.shape, device, out.kq):
         return False
-    out.w, out.K, out.N, out.act = w.data_ptr(), K, N, _ACTS[layer._act_name]
+    out.w, out.K, out.N = w.data_ptr(), K, N
+    out.act = _lib.ACT_RELU if layer._act_name == 'relu' else _lib.ACT_NONE
     if b is not None:
         if layer._bq is None or b.dtype is not torch.float32 or b.device != device or not b.is_contiguous() or b.numel() != N:
             return False
