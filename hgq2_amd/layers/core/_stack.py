@@ -131,7 +131,7 @@ def predict_contraction(layer, x, K, N, out_shape):
 def predict_run(layers, first, x):
     """``(output, index behind the last layer taken)`` for the longest run of layers from ``first`` on that one library call
     covers, or ``None``."""
-    if x.dim() != 2 or not _plain_input(x):
+    if type(x) is not torch.Tensor or x.dim() != 2 or not _plain_input(x):  # (lists and tuples pass between layers too)
         return None
     rows, width = x.shape
     descs = (_lib.StackLayer * _lib.STACK_MAX_LAYERS)()

@@ -6,7 +6,7 @@ import torch
 
 from hgq2_amd import _lib, core, ops
 from hgq2_amd.config import LayerConfigScope
-from hgq2_amd.core import Sequential
+from hgq2_amd.core import Layer, Sequential
 from hgq2_amd.layers import QDense, QEinsumDense
 from hgq2_amd.layers.core import _stack, dense, einsum_dense
 from hgq2_amd.quantizer.internal import FixedPointQuantizerKBI, FixedPointQuantizerKIF
@@ -77,3 +77,24 @@ def test_activations_that_are_not_the_kernels_own_are_applied(kind, routed):
         with torch.no_grad():
             make(activation=act)(x, training=False)
         assert routed.pop()[0][2] == code and not routed
+
+
+class _Split(Layer):
+    def call(self, x, training=None):
+        return [x, x + 1.0] if self.name == 'list' else (x, x + 1.0)
+
+
+class _Join(Layer):
+    def call(self, xs, training=None):
+        return xs[0] + xs[1]
+
+
+@pytest.mark.parametrize('kind', ['list', 'tuple'])
+def test_lists_and_tuples_pass_between_the_layers_of_a_sequence(kind, routed):
+    net = Sequential([_Split(name=kind), _Join(), _dense(3, 4), _Split(name=kind)])
+    x = torch.ones((5, 4))
+    with torch.no_grad():
+        a, b = net(x, training=False)
+        assert len(routed) == 1 and torch.equal(b - a, torch.ones((5, 3)))
+        assert torch.equal(Sequential([_Join()])([x, x], training=False), 2 * x)
+    assert torch.equal(Sequential([_Split(name=kind), _Join()])(x, training=False), 2 * x + 1)
