@@ -111,7 +111,7 @@ def _plain_input(x) -> bool:
 def predict_contraction(layer, x, K, N, out_shape):
     """Output of a contraction layer's whole call - input, kernel, bias and output quantizer, contraction, activation - outside
     training, tracing and gradients as one library call, or ``None``.  ``x`` [..., K] and the output are read as rows."""
-    if not _plain_input(x) or x.shape[0] * K > x.numel():
+    if not _plain_input(x) or x.dim() < 1 or x.numel() % K:  # (what is no whole number of rows is for the layer to refuse)
         return None
     rows, device = x.numel() // K, x.device
     descs = (_lib.StackLayer * 1)()

@@ -98,3 +98,14 @@ def test_lists_and_tuples_pass_between_the_layers_of_a_sequence(kind, routed):
         assert len(routed) == 1 and torch.equal(b - a, torch.ones((5, 3)))
         assert torch.equal(Sequential([_Join()])([x, x], training=False), 2 * x)
     assert torch.equal(Sequential([_Split(name=kind), _Join()])(x, training=False), 2 * x + 1)
+
+
+def test_inputs_that_are_no_whole_number_of_rows_stay_refused(routed):
+    layer = _einsum('bpf,fh->bph', (2, 3), (None, 2, 4), iq=False)
+    for shape in ((2, 9), (2, 3, 3), (2, 11), (1, 7)):
+        for grad in (True, False):
+            with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+                layer(torch.ones(shape), training=False)
+    with torch.no_grad():
+        layer(torch.ones((2, 2, 4)), training=False)
+    assert routed == [[(4, 3, _lib.ACT_NONE)]]
