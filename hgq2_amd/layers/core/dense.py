@@ -70,7 +70,7 @@ class QDense(QLayerBaseSingleInput):
         return tuple(input_shape[:-1]) + (self.units,)
 
     def call(self, inputs, training=None):
-        if training is False and type(self) is QDense and not torch.is_grad_enabled():
+        if training is False and type(self) is QDense and not torch.is_grad_enabled() and inputs.dim() > 0:
             y = predict_contraction(self, inputs, inputs.shape[-1], self.units, tuple(inputs.shape[:-1]) + (self.units,))
             if y is not None:
                 return y

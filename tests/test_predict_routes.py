@@ -109,3 +109,11 @@ def test_inputs_that_are_no_whole_number_of_rows_stay_refused(routed):
     with torch.no_grad():
         layer(torch.ones((2, 2, 4)), training=False)
     assert routed == [[(4, 3, _lib.ACT_NONE)]]
+
+
+def test_a_single_value_without_axes(routed):
+    layer = _dense(3, 1)
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad):
+            assert layer(torch.tensor(2.0), training=False).shape == (3,)
+    assert not routed
