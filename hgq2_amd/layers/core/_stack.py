@@ -20,7 +20,7 @@ def _mode(round_mode, overflow_mode, training, kbi, symmetric):
 def _describe(q, shape, device, out) -> bool:
     """Fill ``out`` with the variables of the quantizer wrapper ``q`` as its call on a tensor of ``shape`` outside training
     uses them; False where that call is anything but one deterministic fixed-point quantizer."""
-    if type(q) is not Quantizer or not q.built or not q.plain:
+    if type(q) is not Quantizer or not q.built or not q.plain or 'call' in q.__dict__:
         return False
     fq = q.quantizer
     kind = type(fq)
@@ -30,7 +30,7 @@ def _describe(q, shape, device, out) -> bool:
         kbi = True
     else:
         return False
-    if not fq.built or fq.stochastic or fq.__dict__.get('call') is not None:
+    if not fq.built or fq.stochastic or 'call' in fq.__dict__:
         return False
     p = fq._parameters
     i, fb, k = p.get('_i'), p.get('_b' if kbi else '_f'), fq._buffers.get('_var_k')

@@ -23,6 +23,7 @@ def routed(monkeypatch):
 
     def layer_path(x, iq, qkernel, qbias, act, training, oq=None, out_shape=None):
         K, N = qkernel.shape
+        x = x if iq is None else iq(x, training=training)
         y = x.reshape(-1, K)[:, :1] * 0.0 + torch.zeros(N)
         return y, act == 'relu', None, False
 
@@ -117,3 +118,18 @@ def test_a_single_value_without_axes(routed):
         with torch.set_grad_enabled(grad):
             assert layer(torch.tensor(2.0), training=False).shape == (3,)
     assert not routed
+
+
+@pytest.mark.parametrize('place', ['_iq', '_kq', '_bq', '_oq'])
+@pytest.mark.parametrize('inner', [False, True])
+def test_replaced_quantizer_calls_run(place, inner, routed):
+    with LayerConfigScope(enable_oq=True):
+        layer = _dense(3, 4)
+    q, seen = getattr(layer, place), []
+    target = q.quantizer if inner else q
+    target.call = lambda x, training=None: seen.append(place) or x
+    x = torch.ones((5, 4))
+    for net in (layer, Sequential([layer])):
+        with torch.no_grad():
+            net(x, training=False)
+    assert seen == [place, place] and not routed
