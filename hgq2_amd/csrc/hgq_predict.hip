@@ -127,8 +127,14 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
             if (cb * 32 < Np) {
                 const float *w = lds + d.off_w[l];
                 const floatx16 zero = {0};
-                const floatx16 acc = mfma_chain_bf16<false, false>(zero, src + (rh * 32 + (lane & 31)) * CHAIN_LD + half, 1,
-                                                                   w + half * Np + cb * 32 + (lane & 31), Np, batches);
+                const float *ap = src + (rh * 32 + (lane & 31)) * CHAIN_LD + half, *bp = w + half * Np + cb * 32 + (lane & 31);
+                floatx16 acc = mfma_chain_bf16<false, false>(zero, ap, 1, bp, Np, batches);
+                // an infinity is not the sum of its bf16 parts (times a part that is zero it is a NaN): such a tile again on
+                // the fp32 instruction
+                bool bad = false;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[r]) < INFINITY);
+                if (__any(bad)) acc = mfma_chain(zero, ap, 1, bp, Np, batches);
                 const int c = cb * 32 + (lane & 31);
                 const float b = w[batches * 16 * Np + c];
                 // the next layer's input quantizer, column c (nothing is read past its table: c < N = next K)

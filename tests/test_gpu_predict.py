@@ -163,3 +163,27 @@ def test_projections_over_positions(T, K, N, H, oq, shared, monkeypatch):
         assert net(x[:0]).shape == (0, T, N, H)
         many = x.repeat(40000 // (37 * T) + 2, 1, 1)  # beyond the rows one launch takes
         assert torch.equal(net(many), _layerwise(net, many, monkeypatch))
+
+
+# widths of the one-launch form and of the tiled products; samples of one bf16 part beside kernels of two (zero parts among them)
+@pytest.mark.parametrize('dims', [(7, 20), (8, 20), (33, 64), (5, 40, 3), (64, 5), (7, 80), (100, 30)])
+def test_infinities_as_in_a_sum_of_products(dims):
+    g = torch.Generator().manual_seed(len(dims) + dims[0])
+    net = _net(dims, iq=False, bias=False)
+    x = torch.round(4 * torch.randn((70, dims[0]), generator=g)) / 4
+    net(x.cuda())
+    for layer in net.layers:
+        layer._kernel.data.copy_(torch.randn(layer._kernel.shape, generator=g) * 0.3)
+        layer.kq.quantizer._b.data.fill_(12.0)
+    x[3, 2], x[40, 1], x[69, 0], x[10, 3] = float('inf'), float('-inf'), float('nan'), float('inf')
+    want = x.double()
+    for layer in net.layers:
+        want = want @ layer.qkernel.detach().double().cpu()
+        if layer._act_name == 'relu':
+            want = torch.where(want > 0, want, torch.zeros_like(want))
+    with torch.no_grad():
+        got = net(x.cuda())
+    got = got.cpu()
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(got), kind(want))
+    assert len(dims) > 2 or torch.isposinf(want).any()
