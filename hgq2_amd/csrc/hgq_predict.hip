@@ -28,6 +28,7 @@ struct ChainDev {
     hgq_stack_layer l[HGQ_STACK_MAX_LAYERS];
     int off_w[HGQ_STACK_MAX_LAYERS];  // kernel [Kp][Np], zero padded (Kp: multiple of 16, Np: of 32), then the bias [Np]
     int n_layers, off_q, off_a;       // off_q: (k, i, f) of the input quantizers, [n_layers][3][64]; off_a: two tiles
+    int bf16;                         // the matrix instruction (hgq_dense_use_bf16_parts)
 };
 
 __device__ __forceinline__ KIF stack_entry(const hgq_stack_quant &q, int e) {
@@ -128,10 +129,11 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
                 const float *w = lds + d.off_w[l];
                 const floatx16 zero = {0};
                 const float *ap = src + (rh * 32 + (lane & 31)) * CHAIN_LD + half, *bp = w + half * Np + cb * 32 + (lane & 31);
-                floatx16 acc = mfma_chain_bf16<false, false>(zero, ap, 1, bp, Np, batches);
+                floatx16 acc = zero;
+                if (d.bf16) acc = mfma_chain_bf16<false, false>(zero, ap, 1, bp, Np, batches);
                 // an infinity is not the sum of its bf16 parts (times a part that is zero it is a NaN): such a tile again on
                 // the fp32 instruction
-                bool bad = false;
+                bool bad = !d.bf16;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[r]) < INFINITY);
                 if (__any(bad)) acc = mfma_chain(zero, ap, 1, bp, Np, batches);
@@ -263,6 +265,7 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
     if (form == 1) {
         ChainDev d = {};
         const int bytes = chain_layout(layers, n_layers, d);
+        d.bf16 = hgq_dense_use_bf16_parts(-1) != 0;
         if (bytes > 64 * 1024) {
             hipError_t e = hipFuncSetAttribute((const void *)stack_chain_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, CHAIN_LDS);
             if (e != hipSuccess) return fail(HGQ_ERR_LAUNCH, "hgq_dense_stack_predict: hipFuncSetAttribute: %s", hipGetErrorString(e));

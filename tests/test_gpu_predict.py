@@ -8,7 +8,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from hgq2_amd import core, ops  # noqa: E402
+from hgq2_amd import _lib, core, ops  # noqa: E402
 from hgq2_amd.config import LayerConfigScope, QuantizerConfigScope  # noqa: E402
 from hgq2_amd.core import Sequential  # noqa: E402
 from hgq2_amd.layers import QDense, QEinsumDense  # noqa: E402
@@ -187,3 +187,25 @@ def test_infinities_as_in_a_sum_of_products(dims):
     for kind in (torch.isnan, torch.isposinf, torch.isneginf):
         assert torch.equal(kind(got), kind(want))
     assert len(dims) > 2 or torch.isposinf(want).any()
+
+
+@pytest.mark.parametrize('K,N', [(8, 5), (48, 64)])
+def test_the_choice_of_matrix_instruction_holds(K, N):
+    # samples of three parts against kernels of one: three rounded sums per product on the bf16 instruction, one on the fp32 one
+    g = torch.Generator().manual_seed(K)
+    net = _net((K, N), iq=False, bias=False)
+    x = torch.randn((500, K), generator=g).cuda()
+    net(x)
+    lib = _lib.load()
+    with torch.no_grad():
+        on = net(x)
+        before = lib.hgq_dense_use_bf16_parts(0)
+        try:
+            off = net(x)
+        finally:
+            lib.hgq_dense_use_bf16_parts(before)
+        w = net.layers[0].qkernel.double()
+        exact, magnitude = (x.double() @ w).relu(), x.abs().double() @ w.abs()
+    for y in (on, off):  # any order of summation, the parts at most nine sums per product
+        assert ((y - exact).abs() <= 2 * (K + 8) * 2.0**-24 * magnitude + 1e-30).all()
+    assert not torch.equal(off, on)
