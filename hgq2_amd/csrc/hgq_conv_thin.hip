@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256, 3) void thin_fwd_kernel(const float *__restric
     const int m = wave * 32 + (lane & 31);
     const FastDiv by_ow((uint32_t)g.OW), by_xwc((uint32_t)xwc);
     const int my = (int)by_ow.div((uint32_t)m), base = m < p.rows * g.OW ? (my * p.xw + m - my * g.OW) * C : 0;
-    float b[KS][NB][8];
+    float b[KS][NB][8], w0 = 0.f;  // w0: zero times every kernel entry, a NaN if one of them is not finite
     int at[KS][8];
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -81,8 +81,10 @@ __global__ __launch_bounds__(256, 3) void thin_fwd_kernel(const float *__restric
             for (int n = 0; n < NB; ++n) {
                 const int f = n * 32 + (lane & 31);
                 b[s][n][u] = k < K && f < F ? w[k * F + f] : 0.f;
+                w0 = __fmaf_rn(b[s][n][u], 0.f, w0);
             }
         }
+    const bool wild_w = __any(!(w0 == 0.f));
     float bv[NB];
 #pragma unroll
     for (int n = 0; n < NB; ++n) bv[n] = bias && n * 32 + (lane & 31) < F ? bias[n * 32 + (lane & 31)] : 0.f;
@@ -106,6 +108,7 @@ __global__ __launch_bounds__(256, 3) void thin_fwd_kernel(const float *__restric
         __syncthreads();
         if (wave * 32 >= n_px) continue;
         floatx16 acc[NB];
+        float sum0 = 0.f;  // zero times this lane's inputs
 #pragma unroll
         for (int n = 0; n < NB; ++n) acc[n] = floatx16{0};
 #pragma unroll
@@ -115,9 +118,23 @@ __global__ __launch_bounds__(256, 3) void thin_fwd_kernel(const float *__restric
             for (int u = 0; u < 8; ++u) {
                 const float v = m < n_px ? xs[at[s][u]] : 0.f;  // (the LDS behind a short band may hold anything)
                 a[u] = 16 * s + 2 * u + 1 < K ? v : (16 * s + 2 * u + half < K ? v : 0.f);
+                sum0 = __fmaf_rn(a[u], 0.f, sum0);
             }
 #pragma unroll
             for (int n = 0; n < NB; ++n) acc[n] = mfma_batch_bf16<false, false>(acc[n], a, b[s][n]);
+        }
+        // (an infinity is not the sum of its bf16 parts)
+        if (wild_w || __any(!(sum0 == 0.f))) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[n] = floatx16{0};
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const float v = m < n_px && 16 * s + 2 * u + half < K ? xs[at[s][u]] : 0.f;
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, b[s][n][u], acc[n], 0, 0, 0);
+                }
         }
         float *out = y + ((int64_t)img * g.OH + oy0) * g.OW * F;
         const int left = n_px * F;

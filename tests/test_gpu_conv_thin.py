@@ -63,3 +63,20 @@ def test_gradients_that_are_not_finite_stay_where_they_belong():
     bad = torch.zeros_like(dx, dtype=torch.bool)
     bad[1, 7:10, 5:8], bad[0, 17:20, 19:22] = True, True
     assert torch.equal(~torch.isfinite(dx), bad) and torch.isinf(dx[1, 7:10, 5:8]).all()
+
+
+# inputs of one bf16 part, kernels of two (zero parts among them): one block of filters and two, one batch of taps and two
+@pytest.mark.parametrize('C,k,F', [(1, 3, 40), (3, 3, 64), (1, 5, 48), (2, 3, 33)])
+def test_infinite_inputs_as_on_the_fp32_instruction(C, k, F):
+    g = torch.Generator().manual_seed(F)
+    x, w = torch.round(4 * torch.randn((2, 12, 15, C), generator=g)) / 4, torch.round(2**12 * torch.randn((k, k, C, F), generator=g)) / 2**12
+    x[0, 5, 5, 0], x[1, 2, 3, C - 1], x[1, 9, 9, 0] = float('inf'), float('-inf'), float('nan')
+    lib = _lib.load()
+    got = ops.conv2d(x.cuda(), w.cuda(), None, (1, 1), 'valid', (1, 1), 0)
+    before = lib.hgq_dense_use_bf16_parts(0)
+    try:
+        want = ops.conv2d(x.cuda(), w.cuda(), None, (1, 1), 'valid', (1, 1), 0)
+    finally:
+        lib.hgq_dense_use_bf16_parts(before)
+    for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(kind(got), kind(want)) and kind(want).any()
