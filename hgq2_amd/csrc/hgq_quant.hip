@@ -347,7 +347,7 @@ __global__ __launch_bounds__(Q1D_BS) void quant_fwd_bwd_pe(const f32x4 *__restri
 // every reduction below), and a workgroup walks a contiguous chunk of rows (forward) or every so many
 // batches (backward) so that a column sees few workgroups - and few atomics - at the end.
 #define QC_U 8
-#define QC_BWD_U 4
+#define QC_BWD_U 4  // (two operands; the next batch's are in flight beside them)
 template <int VEC>
 __device__ __forceinline__ void qc_load(const __amdgpu_buffer_rsrc_t rs, uint32_t off, float *o) {
     if (VEC == 4) {
@@ -1080,7 +1080,7 @@ static bool sliced_bwd_geometry(int64_t n, int64_t bw_size, int64_t bw_inner, bo
     const int64_t cg = vec ? bw_size / 4 : bw_size;
     TX = pow2_floor_le64(cg);
     gx = (cg + TX - 1) / TX;
-    return cols_grid(n / bw_size, bw_size, (256 / TX) * QC_BWD_U, gx, gy, rows_per_wg);
+    return cols_grid(n / bw_size, bw_size, (256 / TX) * QC_U, gx, gy, rows_per_wg);
 }
 
 extern "C" int64_t hgq_quantize_bwd_workspace(int64_t n, int64_t bw_size, int64_t bw_inner) {
@@ -1248,7 +1248,7 @@ extern "C" int hgq_quantize_bwd(const float *dy, const float *x, const void *k, 
         const int TX = pow2_floor_le64(cg), TY = 256 / TX;
         const int64_t gx = (cg + TX - 1) / TX;
         int64_t gy, rows_per_wg;
-        cols_grid(rows, M, TY * QC_BWD_U, gx, gy, rows_per_wg);
+        cols_grid(rows, M, TY * QC_U, gx, gy, rows_per_wg);
         HGQ_DISPATCH_RM_OM(m.round_mode, m.overflow_mode, {
             if (vec)
                 hipLaunchKernelGGL((quant_bwd_cols<RM, OM, 4>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dy, x, k, i, fb, dx, di, dfb, rows, M, TX, mode, (float *)nullptr);

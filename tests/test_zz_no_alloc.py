@@ -79,3 +79,11 @@ def test_static_scratch_entry_point_refuses_what_does_not_fit():
     # a shape the per-column kernels do not take at all is refused as unsupported
     rc = lib.hgq_quantize_bwd_static(_p(z), _p(z), _p(z), _p(z), _p(z), _p(z), _p(z), _p(z), 16, 16, 1, mode, ctypes.c_void_p(0))
     assert rc == _lib.ERR_UNSUPPORTED
+
+
+# columns whose slices just fit the array on 256 CUs, narrow and wide, whole batches of rows and a remainder
+@pytest.mark.parametrize('rows,M', [(4096, 1024), (1024, 4096), (10000, 256), (64, 65536)])
+def test_static_scratch_takes_what_fills_it(rows, M):
+    from hgq2_amd import _lib
+
+    _both(_lib.load(), _lib, torch.device('cuda:0'), rows, M, M, _lib.mode_bits('RND', 'SAT', training=True), True)
