@@ -1178,6 +1178,10 @@ static int fwd_ksplit(int64_t rows, int K, int F) {
 }
 
 
+// A long contraction onto few columns for few rows: a wavefront per row and quarter of k (`skinny_fwd_kernel`)
+static bool skinny_shape(int64_t rows, int K, int F) { return F <= 16 && K >= 1024 && rows <= 16384; }
+bool dense_split_k(int64_t rows, int K, int F) { return skinny_shape(rows, K, F) || fwd_ksplit(rows, K, F) > 1; }
+
 // EBOPs of a convolution: sum over all output pixels and filters of conv(bits_in, bits_ker), and
 // its gradient, without running the convolution:
 //     S[tap, c] = sum of bits_in over the input pixels that tap visits,   Wsum[tap, c] = sum_f bits_ker[tap, c, f]
@@ -1638,8 +1642,8 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
     kchunk = (kchunk + CV_BK - 1) / CV_BK * CV_BK;
     const int nz = (K + kchunk - 1) / kchunk;
     float *dst = nz > 1 ? workspace : y;
-    if (g->kh == 1 && g->kw == 1 && g->sy == 1 && g->sx == 1 && g->py == 0 && g->px == 0 && g->OH == g->H && g->OW == g->W && F <= 16 &&
-        K >= 1024 && rows <= 16384) {
+    if (g->kh == 1 && g->kw == 1 && g->sy == 1 && g->sx == 1 && g->py == 0 && g->px == 0 && g->OH == g->H && g->OW == g->W &&
+        skinny_shape(rows, K, F)) {
         const dim3 grid((unsigned)((rows + SK_ROWS - 1) / SK_ROWS));
 #define HGQ_SKINNY(FV) \
     case FV: hipLaunchKernelGGL((skinny_fwd_kernel<FV>), grid, dim3(1024), 0, s, xq, qw, qb, y, rows, K, act); break

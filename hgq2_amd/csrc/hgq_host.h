@@ -61,6 +61,9 @@ int gemm_parts_dgrad(const float *dy, const float *mask, const float *w, float *
 int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, int64_t rows, int K, int N, int64_t splits,
                      hipStream_t s);
 
+// Dense contractions with few output tiles that hgq_conv2d_fwd (1 x 1) spreads over the device along k as well.
+bool dense_split_k(int64_t rows, int K, int F);
+
 // Convolutions of any geometry on the same kernels (the data gradient: unit stride); `splits`: gemm_parts_splits(pixels, K, F).
 bool conv_parts_shape(const hgq_conv_geom &g, int F);
 int conv_parts_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);

@@ -8,8 +8,8 @@
 //   per kernel entry, then a short matrix-instruction chain per layer; the call takes 75 us, most of it the host's (a launch
 //   per quantizer and contraction, sixteen in all: 512 us).
 // * Wider layers, or many rows: one launch quantizes all kernels and biases into the workspace, one the input; then per layer
-//   a tiled product whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less), or the
-//   streaming kernel of up to 64 x 64.  50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and
+//   a tiled product whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less), the
+//   streaming kernel of up to 64 x 64, or what hgq_conv2d_fwd has for a product of few tiles.  50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and
 //   contraction: 484 us).
 //
 // Arithmetic per value is that of hgq_quantize_fwd and of the layer's own contraction; the variables are quantized again on
@@ -236,6 +236,26 @@ static int64_t image_floats(const hgq_stack_layer *layers, int n) {
     for (int l = 0; l < n; ++l) at += ((int64_t)layers[l].K * layers[l].N + 3) / 4 * 4 + (layers[l].N + 3) / 4 * 4;
     return at;
 }
+// A product of few output tiles behind a long contraction, which one workgroup per tile would leave to a handful of CUs and a
+// chain of tile steps (32 contraction steps each up to 32 columns, 64 beyond): the forms of hgq_conv2d_fwd that spread it along
+// k, from sixteen tile steps on, with the quantizer behind it as a launch of its own.  Tiled product against those, whole
+// calls: 1024 rows of 3872 -> 10 126 / 28 us, 300 of 2048 -> 512 50 / 34 us, 1024 of 520 -> 3 25.0 / 20.4 us; below the line 1024
+// of 512 -> 512 19.4 / 27.1 us, 64 of 600 -> 64 -> 5 23.9 / 26.7 us, 64 of 784 -> 128 -> 10 28.8 / 28.5 us.
+static bool few_tiles(const hgq_stack_layer &h, int64_t rows) {
+    return (h.K > 64 || h.N > 64) && h.K >= (h.N <= 32 ? 512 : 1024) && dense_split_k(rows, h.K, h.N);
+}
+static hgq_conv_geom dense_geom(const hgq_stack_layer &h, int64_t rows) { return {(int)rows, 1, 1, h.K, 1, 1, 1, 1, 0, 0, 1, 1, 1, 1}; }
+// scratch of such products: the partial sums along k and the result that a quantizer reads
+static int64_t few_floats(const hgq_stack_layer *layers, int n, int64_t rows) {
+    int64_t most = 0;
+    for (int l = 0; l < n; ++l) {
+        if (!few_tiles(layers[l], rows)) continue;
+        const hgq_conv_geom g = dense_geom(layers[l], rows);
+        const int64_t w = (rows * layers[l].N + 3) / 4 * 4 + hgq_conv2d_fwd_workspace(&g, layers[l].N);
+        if (w > most) most = w;
+    }
+    return most;
+}
 // an output quantizer the last product's epilogue does not apply (it takes one entry or one per column)
 static bool table_out(const hgq_stack_layer &h) { return h.oq.i && h.oq.size > h.N; }
 // widest tensor that goes into buffer `which` (0: inputs of even layers, 1: of odd layers, and a last output to be quantized)
@@ -253,7 +273,8 @@ using namespace hgq;
 extern "C" int64_t hgq_dense_stack_workspace(const hgq_stack_layer *layers, int n_layers, int64_t rows) {
     const int form = stack_form(layers, n_layers, rows);
     if (form != 2) return form == 1 ? 0 : -1;
-    return image_floats(layers, n_layers) + buffer_floats(layers, n_layers, rows, 0) + buffer_floats(layers, n_layers, rows, 1);
+    return image_floats(layers, n_layers) + buffer_floats(layers, n_layers, rows, 0) + buffer_floats(layers, n_layers, rows, 1) +
+           few_floats(layers, n_layers, rows);
 }
 
 extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_layers, const float *x, float *y, int64_t rows,
@@ -292,7 +313,7 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
     hipLaunchKernelGGL(stack_prep_kernel, dim3((unsigned)gx, (unsigned)items), dim3(256), 0, s, p);
     int rc = check_launch("hgq_dense_stack_predict(kernels)");
     if (rc) return rc;
-    float *buf[2] = {at, at + buffer_floats(layers, n_layers, rows, 0)};
+    float *buf[2] = {at, at + buffer_floats(layers, n_layers, rows, 0)}, *few = buf[1] + buffer_floats(layers, n_layers, rows, 1);
     const float *cur = x;
     if (const hgq_stack_quant &q = layers[0].iq; q.i) {
         if ((rc = hgq_quantize_fwd(x, q.k, q.i, q.fb, buf[0], nullptr, nullptr, rows * layers[0].K, q.size, 1, q.mode, stream))) return rc;
@@ -303,9 +324,16 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
         const bool last = l + 1 == n_layers, later = last && table_out(h);
         float *out = last && !later ? y : buf[(l + 1) & 1];
         const hgq_stack_quant *oq = last ? (h.oq.i && !later ? &h.oq : nullptr) : layers[l + 1].iq.i ? &layers[l + 1].iq : nullptr;
-        rc = !oq && h.K <= 64 && h.N <= 64
-                 ? hgq_qdense_fwd(cur, nullptr, nullptr, nullptr, 0, qw[l], qb[l], out, nullptr, rows, h.K, h.N, h.act, 0, stream)
-                 : gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq);
+        if (few_tiles(h, rows)) {
+            const hgq_conv_geom g = dense_geom(h, rows);
+            float *z = oq ? few : out, *ws = few + (rows * h.N + 3) / 4 * 4;
+            rc = hgq_conv2d_fwd(cur, qw[l], qb[l], z, ws, &g, h.N, h.act, stream);
+            if (!rc && oq) rc = hgq_quantize_fwd(z, oq->k, oq->i, oq->fb, out, nullptr, nullptr, rows * h.N, oq->size, 1, oq->mode, stream);
+        } else if (!oq && h.K <= 64 && h.N <= 64) {
+            rc = hgq_qdense_fwd(cur, nullptr, nullptr, nullptr, 0, qw[l], qb[l], out, nullptr, rows, h.K, h.N, h.act, 0, stream);
+        } else {
+            rc = gemm_parts_fwd(cur, qw[l], qb[l], out, rows, h.K, h.N, h.act, s, oq);
+        }
         if (rc) return rc;
         if (later) return hgq_quantize_fwd(out, h.oq.k, h.oq.i, h.oq.fb, y, nullptr, nullptr, rows * h.N, h.oq.size, 1, h.oq.mode, stream);
         cur = out;

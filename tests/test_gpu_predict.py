@@ -209,3 +209,60 @@ def test_the_choice_of_matrix_instruction_holds(K, N):
     for y in (on, off):  # any order of summation, the parts at most nine sums per product
         assert ((y - exact).abs() <= 2 * (K + 8) * 2.0**-24 * magnitude + 1e-30).all()
     assert not torch.equal(off, on)
+
+
+# long contractions onto few columns or few rows: a wavefront per row, a split along k with and without a quantizer behind it,
+# first, middle and last layer, output quantizer by column and by position
+@pytest.mark.parametrize('dims,rows', [((3872, 10), 1), ((3872, 10), 1024), ((1025, 16), 7), ((1024, 17), 130), ((513, 3), 20000), ((700, 20, 5), 65),
+                                       ((70, 1100, 33), 3), ((1030, 70, 1500, 40, 2), 200), ((2048, 512), 64), ((511, 9), 31), ((1023, 65), 12)])
+def test_long_contractions(dims, rows, monkeypatch):
+    g = torch.Generator().manual_seed(rows)
+    net = _net(dims)
+    x = torch.randn((max(rows, 200), dims[0]), generator=g).cuda()
+    net(x)
+    _spread(net, g)
+    trace_minmax(net, x)
+    taken, inner = [], ops.dense_stack_predict
+    monkeypatch.setattr(ops, 'dense_stack_predict', lambda *a: taken.append(a[2]) or inner(*a))
+    with torch.no_grad():
+        got = net(x[:rows])
+    assert taken and torch.equal(got, _layerwise(net, x[:rows], monkeypatch))
+
+
+@pytest.mark.parametrize('shared', [None, (0, 1)])
+@pytest.mark.parametrize('T,K,N', [(1, 2000, 8), (3, 1500, 40)])
+def test_long_contractions_with_an_output_quantizer(T, K, N, shared, monkeypatch):
+    kw = dict(homogeneous_axis=shared, heterogeneous_axis=None) if shared else {}
+    g = torch.Generator().manual_seed(K)
+    with QuantizerConfigScope(place='all', default_q_type='kbi', overflow_mode='SAT_SYM'), \
+            QuantizerConfigScope(place='datalane', default_q_type='kif', overflow_mode='WRAP', **kw), LayerConfigScope(enable_ebops=False):
+        net = QEinsumDense('btf,fh->bth', output_shape=(T, N), bias_axes='h', enable_oq=True)
+    core.set_default_device('cuda')
+    x = torch.randn((37, T, K), generator=g).cuda()
+    net(x)
+    _spread(net, g)
+    trace_minmax(net, x)
+    with torch.no_grad():
+        got = net(x)
+    assert torch.equal(got, _layerwise(net, x, monkeypatch))
+
+
+def test_long_contractions_are_split_along_k():
+    """The workspace shows the form: partial sums along k where a product has few tiles and many steps, none elsewhere."""
+    lib = _lib.load()
+    one = torch.ones(1, device='cuda')
+    u8 = torch.ones(1, dtype=torch.uint8, device='cuda')
+
+    def floats(rows, K, N):
+        d = (_lib.StackLayer * 1)()
+        d[0].w, d[0].K, d[0].N = one.data_ptr(), K, N
+        d[0].kq.k, d[0].kq.i, d[0].kq.fb, d[0].kq.size, d[0].kq.inner = u8.data_ptr(), one.data_ptr(), one.data_ptr(), 1, 1
+        return lib.hgq_dense_stack_workspace(d, 1, rows)
+
+    def image(K, N):
+        return (K * N + 3) // 4 * 4 + (N + 3) // 4 * 4
+
+    for rows, K, N in ((64, 2048, 512), (1, 4096, 100), (300, 600, 20)):
+        assert floats(rows, K, N) >= image(K, N) + 2 * rows * N
+    for rows, K, N in ((1024, 512, 512), (64, 600, 64), (50000, 2048, 512)):
+        assert floats(rows, K, N) == image(K, N)
