@@ -5,8 +5,8 @@
 // * Every width up to 64 (`stack_chain_kernel`): ONE launch.  A workgroup quantizes all kernels and biases into LDS, then
 //   takes tiles of 64 samples through every layer; between layers a tile stays in LDS and the next layer's input quantizer
 //   runs on the accumulator registers.  One event through 16-64-32-32-5 is bound by latency: four loads and one rounding
-//   per kernel entry, then a short matrix-instruction chain per layer; the call takes 75 us, most of it the host's (a launch
-//   per quantizer and contraction, sixteen in all: 512 us).
+//   per kernel entry, then a short matrix-instruction chain per layer (19 us); the call takes 75 us, most of it the host's (a
+//   launch per quantizer and contraction, sixteen in all: 512 us).
 // * Wider layers, or many rows: one launch quantizes all kernels and biases into the workspace, one the input; then per layer
 //   a tiled product whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less), the
 //   streaming kernel of up to 64 x 64, or what hgq_conv2d_fwd has for a product of few tiles.  50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and
@@ -22,14 +22,22 @@ namespace hgq {
 #define CHAIN_BM 64
 #define CHAIN_LD 65   // odd row stride: the 32 rows of an operand read fall into different banks
 #define CHAIN_LDS (160 * 1024)  // of a CU; seven layers of 64 x 64 fit
-#define CHAIN_NT 256  // four wavefronts: row half x column half of a tile
+// Eight wavefronts stage, quantize and store; four of them contract, row half x column half of a tile.  Quantizing the kernels is
+// what a call of few samples waits for, two wavefronts per SIMD issue it nearly twice as fast as one: 64 x 64 on one sample
+// 14.9 -> 10.4 us, seven such layers 67.3 -> 44.6 us, 16-64-32-32-5 22.0 -> 19.3 us.  (Sixteen wavefronts: 8.9, 35.7, 19.2 us, and
+// one workgroup per CU instead of two: 39 against 23 us for the last on 32 768 samples.)
+#define CHAIN_NT 512
 
 struct ChainDev {
     hgq_stack_layer l[HGQ_STACK_MAX_LAYERS];
     int off_w[HGQ_STACK_MAX_LAYERS];  // kernel [Kp][Np], zero padded (Kp: multiple of 16, Np: of 32), then the bias [Np]
     int n_layers, off_q, off_a;       // off_q: (k, i, f) of the input quantizers, [n_layers][3][64]; off_a: two tiles
-    int bf16;                         // the matrix instruction (hgq_dense_use_bf16_parts)
+    uint32_t how;                     // two bits per layer, CHAIN_*
 };
+// How a layer multiplies.  An infinity is not the sum of its bf16 parts (times a part that is zero it is a NaN): where an operand
+// may hold one a tile whose sums are not all finite is contracted again on the fp32 instruction.  A quantizer outside training
+// leaves none: it saturates them or wraps them to NaNs.
+enum { CHAIN_BF16 = 0, CHAIN_CHECKED = 1, CHAIN_FP32 = 2 };
 
 __device__ __forceinline__ KIF stack_entry(const hgq_stack_quant &q, int e) {
     const Mode m(q.mode);
@@ -125,18 +133,19 @@ __global__ __launch_bounds__(CHAIN_NT) void stack_chain_kernel(const ChainDev d,
             float *dst = tiles + ((l + 1) & 1) * CHAIN_BM * CHAIN_LD;
             const bool last = l + 1 == L;
             __syncthreads();  // the source tile is complete
-            if (cb * 32 < Np) {
+            if (wave < 4 && cb * 32 < Np) {
                 const float *w = lds + d.off_w[l];
                 const floatx16 zero = {0};
                 const float *ap = src + (rh * 32 + (lane & 31)) * CHAIN_LD + half, *bp = w + half * Np + cb * 32 + (lane & 31);
+                const uint32_t how = (d.how >> (2 * l)) & 3u;
                 floatx16 acc = zero;
-                if (d.bf16) acc = mfma_chain_bf16<false, false>(zero, ap, 1, bp, Np, batches);
-                // an infinity is not the sum of its bf16 parts (times a part that is zero it is a NaN): such a tile again on
-                // the fp32 instruction
-                bool bad = !d.bf16;
+                if (how != CHAIN_FP32) acc = mfma_chain_bf16<false, false>(zero, ap, 1, bp, Np, batches);
+                if (how != CHAIN_BF16) {
+                    bool bad = how == CHAIN_FP32;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[r]) < INFINITY);
-                if (__any(bad)) acc = mfma_chain(zero, ap, 1, bp, Np, batches);
+                    for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[r]) < INFINITY);
+                    if (__any(bad)) acc = mfma_chain(zero, ap, 1, bp, Np, batches);
+                }
                 const int c = cb * 32 + (lane & 31);
                 const float b = w[batches * 16 * Np + c];
                 // the next layer's input quantizer, column c (nothing is read past its table: c < N = next K)
@@ -224,9 +233,11 @@ static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
     ChainDev d;
     wide = wide && hgq_dense_use_bf16_parts(-1) != 0;
     chain = chain && chain_layout(layers, n, d) <= CHAIN_LDS;
-    // One launch where the host and the launches are what a call costs.  Many rows: the streaming kernels move them faster -
-    // an attention block of three heads on 400 000 rows, four projections with tables each way: 1293 us on this kernel, 949 us on those; four
-    // layers without tables on 65 536 rows still finish before the host does (76 us).
+    // One launch where the host and the launches are what a call costs, and as long as it is not the slower one on the device
+    // either.  Device time of recorded calls, one launch against a launch per layer: 16-64-32-32-5 on 65 536 rows 32 / 54 us,
+    // seven layers of 64 units 118 / 117 us; 64 onto 64 with tables for input and output on 32 768 rows 21.8 / 25.4 us, on
+    // 65 536 36.3 / 30.9 us.  (On a few rows 64 onto 64 alone is 10.4 / 8.5 us, with both tables 16.7 / 11.3 us, and an eager call
+    // of two or three launches more takes the host 7 us longer.)
     if (chain && (!wide || rows <= (tables ? 32768 : 65536))) return 1;
     return wide ? 2 : 0;
 }
@@ -286,7 +297,11 @@ extern "C" int hgq_dense_stack_predict(const hgq_stack_layer *layers, int n_laye
     if (form == 1) {
         ChainDev d = {};
         const int bytes = chain_layout(layers, n_layers, d);
-        d.bf16 = hgq_dense_use_bf16_parts(-1) != 0;
+        for (int l = 0; l < n_layers; ++l) {
+            const Mode mi(layers[l].iq.mode), mk(layers[l].kq.mode);
+            const bool open = !layers[l].iq.i || (mi.overflow_mode == HGQ_WRAP && mi.training) || (mk.overflow_mode == HGQ_WRAP && mk.training);
+            d.how |= (uint32_t)(!hgq_dense_use_bf16_parts(-1) ? CHAIN_FP32 : open ? CHAIN_CHECKED : CHAIN_BF16) << (2 * l);
+        }
         if (bytes > 64 * 1024) {
             hipError_t e = hipFuncSetAttribute((const void *)stack_chain_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, CHAIN_LDS);
             if (e != hipSuccess) return fail(HGQ_ERR_LAUNCH, "hgq_dense_stack_predict: hipFuncSetAttribute: %s", hipGetErrorString(e));
