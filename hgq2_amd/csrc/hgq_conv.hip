@@ -1515,9 +1515,23 @@ static bool bwd_smallc_ok(const hgq_conv_geom &g, int F) {
            bwd_smallc_lds(g, F) <= 64 * 1024 && (int64_t)g.B * g.OH * g.OW * F * 4 < (1ll << 31) &&
            (int64_t)g.B * g.H * g.W * g.C * 4 < (1ll << 31);
 }
-static int bwd_smallc_grid(const hgq_conv_geom &g) {
-    const int64_t tiles = (int64_t)g.B * ((g.H + SC_TH - 1) / SC_TH) * ((g.W + SC_TW - 1) / SC_TW);
-    return persistent_grid(tiles, 3);
+static int64_t bwd_smallc_tiles(const hgq_conv_geom &g) {
+    return (int64_t)g.B * ((g.H + SC_TH - 1) / SC_TH) * ((g.W + SC_TW - 1) / SC_TW);
+}
+static int bwd_smallc_grid(const hgq_conv_geom &g) { return persistent_grid(bwd_smallc_tiles(g), 3); }
+// The backward pass over few input values per pixel on the matrix cores (conv_thin_bwd) or with multiply-adds per pixel and
+// filter (bwd_smallc_kernel, 3 x 3).  The first takes its two workgroups per CU about 4.7 us a round whatever the filters (they
+// are padded to 32), and wide rows leave it short bands; the second's three take 5 us and 0.14 us per channel and filter.
+// Measured over 16 - 1024 images of 12 - 64 pixels, 1 - 3 channels, 1 - 32 filters, with and without a pooling behind: never
+// more than a quarter slower than the better one, 0.4 % on average.  1024 x 28 x 28 x 1 -> 8 behind a pooling 55.5 us on the matrix cores,
+// 33.9 us pixel by pixel; -> 32 54 and 57 us; 1024 x 32 x 32 x 1 -> 8 68.3 and 35.6 us; 300 x 24 x 24 x 3 -> 32 26.0 and 46.9 us.
+static bool thin_bwd_ok(const hgq_conv_geom &g, int F) {
+    if (!conv_thin_bwd_ok(g, F)) return false;
+    if (g.kh != 3 || !bwd_smallc_ok(g, F)) return true;
+    const int cap = persistent_grid(1 << 30, 1);
+    const double thin = 4.7 * (double)((conv_thin_bwd_tiles(g) + 2 * cap - 1) / (2 * cap));
+    const double rounds = (double)bwd_smallc_tiles(g) / (3 * cap);
+    return thin <= (rounds > 1.0 ? rounds : 1.0) * (5.0 + 0.5 * g.C + 0.14 * g.C * F);
 }
 #define HGQ_SMALLC_DISPATCH(CALL) \
     do { \
@@ -1699,7 +1713,7 @@ extern "C" int64_t hgq_conv2d_bwd_workspace(const hgq_conv_geom *g, int F) {
     const WgradCfg c = wgrad_cfg(K, F);
     int64_t slices = wgrad_slices(*g, F, rows, c);
     if (bwd_smallc_ok(*g, F) && bwd_smallc_grid(*g) > slices) slices = bwd_smallc_grid(*g);
-    if (conv_thin_bwd_ok(*g, F) && conv_thin_slices(*g) > slices) slices = conv_thin_slices(*g);
+    if (thin_bwd_ok(*g, F) && conv_thin_slices(*g) > slices) slices = conv_thin_slices(*g);
     if (conv_patch_wgrad_ok(*g, F) && conv_patch_wgrad_slices(*g, F) > slices) slices = conv_patch_wgrad_slices(*g, F);
     return slices * ((int64_t)K * F + F);
 }
@@ -1716,7 +1730,7 @@ extern "C" int64_t hgq_conv2d_bwd_slice_count(const hgq_conv_geom *g, int F) {
     if (check_geom(g, F, "hgq_conv2d_bwd_slice_count")) return -1;
     const int64_t rows = (int64_t)g->B * g->OH * g->OW;
     if (rows == 0) return 1;
-    if (conv_thin_bwd_ok(*g, F)) return conv_thin_slices(*g);
+    if (thin_bwd_ok(*g, F)) return conv_thin_slices(*g);
     if (bwd_smallc_ok(*g, F)) return bwd_smallc_grid(*g);
     if (conv_patch_wgrad_ok(*g, F)) return conv_patch_wgrad_slices(*g, F);
     const WgradCfg c = wgrad_cfg(g->kh * g->kw * g->C, F);
@@ -1747,7 +1761,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
     const float *mask = (act == HGQ_ACT_RELU || dyp) ? y : nullptr;
     if (dyp && !(hgq_conv2d_maxpool_bwd_supported(g, F) && aligned16(dyp) && (code ? ((uintptr_t)code & 3u) == 0 : aligned16(y))))
         return fail(HGQ_ERR_UNSUPPORTED, "hgq_conv2d_maxpool_bwd: shape or alignment not supported (ask hgq_conv2d_maxpool_bwd_supported)");
-    if (conv_thin_bwd_ok(*g, F)) {
+    if (thin_bwd_ok(*g, F)) {
         const bool want_w = dqw || dqb;
         if (want_w && !workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
         if ((rc = conv_thin_bwd(dy, mask, dyp, code, xq, qw, dxq, want_w ? workspace : nullptr, *g, F, act, s))) return rc;

@@ -469,6 +469,7 @@ bool conv_thin_bwd_ok(const hgq_conv_geom &g, int F) {
     const ThinPlan p = bwd_plan(g);
     return (p.bands == 1 ? g.OH : p.rows + g.kh - 1) * p.xw <= 256 && bwd_lds(F, p) <= 120 * 1024 && (int64_t)p.rows * g.W * g.C < (1 << 20);
 }
+int64_t conv_thin_bwd_tiles(const hgq_conv_geom &g) { return bwd_plan(g).tiles; }
 int conv_thin_slices(const hgq_conv_geom &g) { return persistent_grid(bwd_plan(g).tiles, 2); }
 
 int conv_thin_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s) {

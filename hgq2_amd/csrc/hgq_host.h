@@ -70,10 +70,11 @@ int conv_parts_fwd(const float *x, const float *w, const float *bias, float *y, 
 int conv_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, const hgq_conv_geom &g, int F, hipStream_t s);
 int conv_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, const hgq_conv_geom &g, int F, int64_t splits, hipStream_t s);
 
-// Convolutions over few input values per pixel (hgq_conv_thin.hip): which shapes, the slices the backward pass leaves
-// ([K F + F] each), forward, and data + weight + bias gradient in one pass.
+// Convolutions over few input values per pixel (hgq_conv_thin.hip): which shapes, the bands of rows the backward pass works
+// in, the slices it leaves ([K F + F] each), forward, and data + weight + bias gradient in one pass.
 bool conv_thin_fwd_ok(const hgq_conv_geom &g, int F);
 bool conv_thin_bwd_ok(const hgq_conv_geom &g, int F);
+int64_t conv_thin_bwd_tiles(const hgq_conv_geom &g);
 int conv_thin_slices(const hgq_conv_geom &g);
 int conv_thin_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);
 int conv_thin_bwd(const float *dy, const float *mask, const float *dyp, const uint8_t *code, const float *x, const float *w, float *dx,
