@@ -1525,8 +1525,8 @@ static int bwd_smallc_grid(const hgq_conv_geom &g) { return persistent_grid(bwd_
 // Measured over 16 - 1024 images of 12 - 64 pixels, 1 - 3 channels, 1 - 32 filters, with and without a pooling behind: never
 // more than a quarter slower than the better one, 0.4 % on average.  1024 x 28 x 28 x 1 -> 8 behind a pooling 55.5 us on the matrix cores,
 // 33.9 us pixel by pixel; -> 32 54 and 57 us; 1024 x 32 x 32 x 1 -> 8 68.3 and 35.6 us; 300 x 24 x 24 x 3 -> 32 26.0 and 46.9 us.
-static bool thin_bwd_ok(const hgq_conv_geom &g, int F) {
-    if (!conv_thin_bwd_ok(g, F)) return false;
+static bool thin_bwd_shape(const hgq_conv_geom &g, int F) {
+    if (!conv_thin_bwd_shape(g, F)) return false;
     if (g.kh != 3 || !bwd_smallc_ok(g, F)) return true;
     const int cap = persistent_grid(1 << 30, 1);
     const double thin = 4.7 * (double)((conv_thin_bwd_tiles(g) + 2 * cap - 1) / (2 * cap));
@@ -1547,14 +1547,24 @@ static bool dense_shape(const hgq_conv_geom &g, int F) {
     return g.kh == 1 && g.kw == 1 && g.sy == 1 && g.sx == 1 && g.py == 0 && g.px == 0 && g.OH == g.H && g.OW == g.W &&
            gemm_parts_shape((int64_t)g.B * g.H * g.W, g.C, F);
 }
-// ... and its products run on the bf16-part kernels of hgq_gemm.hip unless the fp32 instruction was asked for
-static bool dense_parts(const hgq_conv_geom &g, int F) { return dense_shape(g, F) && hgq_dense_use_bf16_parts(-1) != 0; }
+// The bf16-part kernels of hgq_gemm.hip and hgq_conv_thin.hip run unless the fp32 instruction was asked for.  The choice is
+// process-wide and another thread may change it between a caller's question for slices or workspace and its launch: slices
+// are a function of the shape alone, and either instruction's kernels fill as many.
+static bool parts_on() { return hgq_dense_use_bf16_parts(-1) != 0; }
 // The tiled product gathers the weight gradient's source element by element, for any depth; where four channels make a 128-bit
 // gather wgrad_vec_kernel is the faster one (300 x 11 x 11, 3 x 3, 40 -> 40: 21 against 38 us; 1024 x 13 x 13, 37 -> 37: all
 // gradients 382 -> 220 us with the tiled product).
-static bool wgrad_parts(const hgq_conv_geom &g, int F) { return g.C % 4 != 0 && conv_parts_shape(g, F); }
-static int64_t wgrad_slices(const hgq_conv_geom &g, int F, int64_t rows, const WgradCfg &c) {
-    return dense_shape(g, F) || wgrad_parts(g, F) ? gemm_parts_splits(rows, g.kh * g.kw * g.C, F) : wgrad_splits(rows, c.n_kt * c.n_nt);
+static bool wgrad_parts_shape(const hgq_conv_geom &g, int F) { return g.C % 4 != 0 && conv_parts_shape(g, F); }
+// slices of the weight gradient where no kernel does all gradients in one pass
+static int64_t wgrad_slices(const hgq_conv_geom &g, int F) {
+    const int64_t rows = (int64_t)g.B * g.OH * g.OW;
+    const int K = g.kh * g.kw * g.C;
+    if (conv_patch_wgrad_shape(g, F)) return conv_patch_wgrad_slices(g, F);
+    const WgradCfg c = wgrad_cfg(K, F);
+    return dense_shape(g, F) || wgrad_parts_shape(g, F) ? gemm_parts_splits(rows, K, F) : wgrad_splits(rows, c.n_kt * c.n_nt);
+}
+static int64_t bwd_slices(const hgq_conv_geom &g, int F) {
+    return thin_bwd_shape(g, F) ? conv_thin_slices(g) : bwd_smallc_ok(g, F) ? bwd_smallc_grid(g) : wgrad_slices(g, F);
 }
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1668,7 +1678,7 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
 #undef HGQ_SKINNY
         return check_launch("hgq_conv2d_fwd(few filters, long contraction)");
     }
-    if (nz == 1 && dense_parts(*g, F)) return gemm_parts_fwd(xq, qw, qb, y, rows, K, F, act, s);
+    if (nz == 1 && dense_shape(*g, F) && parts_on()) return gemm_parts_fwd(xq, qw, qb, y, rows, K, F, act, s);
     if (fwd_smallc_ok(*g, F)) {
         const int tiles_x = (g->OW + SC_TW - 1) / SC_TW, tiles_y = (g->OH + SC_TH - 1) / SC_TH;
         const dim3 grid((unsigned)persistent_grid((int64_t)g->B * tiles_x * tiles_y, 8));
@@ -1687,7 +1697,7 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
     if (nz == 1 && conv_thin_fwd_ok(*g, F)) return conv_thin_fwd(xq, qw, qb, y, *g, F, act, s);
     if (nz == 1 && aligned16(xq) && conv_patch_ok(0, *g, F)) return conv_patch_launch(0, xq, nullptr, qw, qb, y, *g, F, act, s);
     // (300 x 11 x 11, 3 x 3, 40 -> 40: 22 -> 15 us; 1024 x 13 x 13, 37 -> 37: 135 -> 51 us against the implicit GEMM below)
-    if (nz == 1 && conv_parts_shape(*g, F)) return conv_parts_fwd(xq, qw, qb, y, *g, F, act, s);
+    if (nz == 1 && parts_on() && conv_parts_shape(*g, F)) return conv_parts_fwd(xq, qw, qb, y, *g, F, act, s);
     const bool vec = g->C % 4 == 0 && aligned16(xq) && (int64_t)g->B * g->H * g->W * g->C * 4 < (1ll << 31);
     if (F <= 32) {
         const dim3 grid((unsigned)persistent_grid((rows + 127) / 128, vec ? 3 : 8), 1, (unsigned)nz);
@@ -1708,14 +1718,7 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
 
 extern "C" int64_t hgq_conv2d_bwd_workspace(const hgq_conv_geom *g, int F) {
     if (check_geom(g, F, "hgq_conv2d_bwd_workspace")) return -1;
-    const int64_t rows = (int64_t)g->B * g->OH * g->OW;
-    const int K = g->kh * g->kw * g->C;
-    const WgradCfg c = wgrad_cfg(K, F);
-    int64_t slices = wgrad_slices(*g, F, rows, c);
-    if (bwd_smallc_ok(*g, F) && bwd_smallc_grid(*g) > slices) slices = bwd_smallc_grid(*g);
-    if (thin_bwd_ok(*g, F) && conv_thin_slices(*g) > slices) slices = conv_thin_slices(*g);
-    if (conv_patch_wgrad_ok(*g, F) && conv_patch_wgrad_slices(*g, F) > slices) slices = conv_patch_wgrad_slices(*g, F);
-    return slices * ((int64_t)K * F + F);
+    return bwd_slices(*g, F) * ((int64_t)g->kh * g->kw * g->C * F + F);
 }
 
 extern "C" int hgq_conv2d_maxpool_bwd_supported(const hgq_conv_geom *g, int F) {
@@ -1728,13 +1731,7 @@ extern "C" int hgq_conv2d_maxpool_bwd_supported(const hgq_conv_geom *g, int F) {
 
 extern "C" int64_t hgq_conv2d_bwd_slice_count(const hgq_conv_geom *g, int F) {
     if (check_geom(g, F, "hgq_conv2d_bwd_slice_count")) return -1;
-    const int64_t rows = (int64_t)g->B * g->OH * g->OW;
-    if (rows == 0) return 1;
-    if (thin_bwd_ok(*g, F)) return conv_thin_slices(*g);
-    if (bwd_smallc_ok(*g, F)) return bwd_smallc_grid(*g);
-    if (conv_patch_wgrad_ok(*g, F)) return conv_patch_wgrad_slices(*g, F);
-    const WgradCfg c = wgrad_cfg(g->kh * g->kw * g->C, F);
-    return wgrad_slices(*g, F, rows, c);
+    return (int64_t)g->B * g->OH * g->OW == 0 ? 1 : bwd_slices(*g, F);
 }
 
 // reduce: the slices of the kernel / bias gradient are summed into dqw / dqb; otherwise they stay in `workspace`
@@ -1761,7 +1758,8 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
     const float *mask = (act == HGQ_ACT_RELU || dyp) ? y : nullptr;
     if (dyp && !(hgq_conv2d_maxpool_bwd_supported(g, F) && aligned16(dyp) && (code ? ((uintptr_t)code & 3u) == 0 : aligned16(y))))
         return fail(HGQ_ERR_UNSUPPORTED, "hgq_conv2d_maxpool_bwd: shape or alignment not supported (ask hgq_conv2d_maxpool_bwd_supported)");
-    if (thin_bwd_ok(*g, F)) {
+    const bool thin = thin_bwd_shape(*g, F), parts = parts_on();
+    if (thin && parts) {
         const bool want_w = dqw || dqb;
         if (want_w && !workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
         if ((rc = conv_thin_bwd(dy, mask, dyp, code, xq, qw, dxq, want_w ? workspace : nullptr, *g, F, act, s))) return rc;
@@ -1771,7 +1769,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
         const bool want_w = dqw || dqb;
         if (want_w && !workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
         const int tiles_x = (g->W + SC_TW - 1) / SC_TW, tiles_y = (g->H + SC_TH - 1) / SC_TH;
-        const int grid = bwd_smallc_grid(*g);
+        const int grid = thin ? conv_thin_slices(*g) : bwd_smallc_grid(*g);
         const size_t lds = bwd_smallc_lds(*g, F);
         const int vec = F % 4 == 0 && aligned16(dy) && (!mask || aligned16(mask));
 #define HGQ_BWD_SC(KH, KW, CC) \
@@ -1782,7 +1780,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
         if (want_w && reduce) return reduce_parts(workspace, grid, KF + F, dqw, KF, dqb, (int64_t)F, nullptr, 0, s);
         return HGQ_OK;
     }
-    if (dense_parts(*g, F)) {
+    if (dense_shape(*g, F) && parts) {
         const float *zmask = act == HGQ_ACT_RELU ? mask : nullptr;
         if (dxq && (rc = gemm_parts_dgrad(dy, zmask, qw, dxq, rows, K, F, s))) return rc;
         if (!dqw && !dqb) return HGQ_OK;
@@ -1814,7 +1812,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
 #undef HGQ_DG
         } else if (aligned16(dy) && (!mask || aligned16(mask)) && conv_patch_ok(1, *g, F)) {
             if ((rc = conv_patch_launch(1, dy, mask, qw, nullptr, dxq, *g, F, act, s))) return rc;
-        } else if (g->sy == 1 && g->sx == 1 && conv_parts_shape(*g, F)) {  // 300 x 11 x 11, 3 x 3, 40 -> 40: 50 -> 27 us
+        } else if (g->sy == 1 && g->sx == 1 && parts && conv_parts_shape(*g, F)) {  // 300 x 11 x 11, 3 x 3, 40 -> 40: 50 -> 27 us
             if ((rc = conv_parts_dgrad(dy, act == HGQ_ACT_RELU ? mask : nullptr, qw, dxq, *g, F, s))) return rc;
         } else {
             const bool vec = F % 4 == 0 && aligned16(dy) && (!mask || aligned16(mask)) && rows * F * 4 < (1ll << 31);
@@ -1831,25 +1829,24 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
     if (dqw || dqb) {
         if (!workspace) return fail(HGQ_ERR_ARG, "hgq_conv2d_bwd: null workspace");
         const int64_t M = KF + F;
-        // small feature maps: both operands of a band of an image staged once in LDS (the slice count is a function of the
-        // shape alone, so operands that are not 16-byte aligned keep it and go through the gathered kernels below)
-        const bool patch_shape = conv_patch_wgrad_ok(*g, F);
-        const int64_t patch_slices = patch_shape ? conv_patch_wgrad_slices(*g, F) : 0;
-        if (patch_shape && aligned16(xq) && aligned16(dy) && (!mask || aligned16(mask))) {
+        int64_t splits = thin ? conv_thin_slices(*g) : wgrad_slices(*g, F);
+        const bool patch_shape = !thin && conv_patch_wgrad_shape(*g, F);
+        // small feature maps: both operands of a band of an image staged once in LDS
+        if (patch_shape && parts && aligned16(xq) && aligned16(dy) && (!mask || aligned16(mask))) {
             if ((rc = conv_patch_wgrad_launch(xq, dy, mask, workspace, *g, F, act, s))) return rc;
-            if (reduce && (rc = reduce_parts(workspace, (int)patch_slices, M, dqw, KF, dqb, (int64_t)F, nullptr, 0, s))) return rc;
+            if (reduce && (rc = reduce_parts(workspace, (int)splits, M, dqw, KF, dqb, (int64_t)F, nullptr, 0, s))) return rc;
             return HGQ_OK;
         }
-        const WgradCfg c = wgrad_cfg(K, F);
-        int64_t splits = wgrad_slices(*g, F, rows, c);
-        if (!patch_shape && wgrad_parts(*g, F)) {
+        if (!thin && !patch_shape && parts && wgrad_parts_shape(*g, F)) {
             if ((rc = conv_parts_wgrad(xq, dy, act == HGQ_ACT_RELU ? mask : nullptr, workspace, *g, F, splits, s))) return rc;
             return reduce ? reduce_parts(workspace, (int)splits, M, dqw, KF, dqb, (int64_t)F, nullptr, 0, s) : HGQ_OK;
         }
-        if (patch_shape) {
-            if (splits > patch_slices) splits = patch_slices;
-            if (splits < patch_slices && !reduce && (rc = fill_f32(workspace + splits * M, 0.f, (patch_slices - splits) * M, s))) return rc;
-        }
+        // the gathered kernels below fill no more slices than they have rows for; a caller who reduces them itself finds zeros
+        // in the rest
+        const WgradCfg c = wgrad_cfg(K, F);
+        const int64_t all = splits, most = wgrad_splits(rows, c.n_kt * c.n_nt);
+        if (splits > most) splits = most;
+        if (splits < all && !reduce && (rc = fill_f32(workspace + splits * M, 0.f, (all - splits) * M, s))) return rc;
         int64_t chunk = (rows + splits - 1) / splits;
         chunk = (chunk + 127) / 128 * 128;
         const dim3 grid((unsigned)(c.n_kt * c.n_nt), (unsigned)splits);

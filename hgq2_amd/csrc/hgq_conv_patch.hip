@@ -736,10 +736,10 @@ static bool plan_wgrad(const hgq_conv_geom &g, int F, WgPlan &p, size_t &lds) {
     return false;
 }
 
-bool conv_patch_wgrad_ok(const hgq_conv_geom &g, int F) {
+bool conv_patch_wgrad_shape(const hgq_conv_geom &g, int F) {
     WgPlan p;
     size_t lds;
-    return hgq_dense_use_bf16_parts(-1) != 0 && plan_wgrad(g, F, p, lds);
+    return plan_wgrad(g, F, p, lds);
 }
 
 int conv_patch_wgrad_slices(const hgq_conv_geom &g, int F) {

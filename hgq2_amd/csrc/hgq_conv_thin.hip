@@ -37,7 +37,7 @@ static bool thin_shape(const hgq_conv_geom &g, int F) {
     const int K = g.kh * g.kw * g.C;
     return ((g.kh == 3 && g.kw == 3) || (g.kh == 5 && g.kw == 5)) && K <= 31 && F >= 1 && F <= 64 && g.sy == 1 && g.sx == 1 && g.dly == 1 &&
            g.dlx == 1 && g.py < g.kh && g.px < g.kw && g.OH <= g.H + g.py && g.OW <= g.W + g.px && g.OW + g.kw - 1 >= g.W + g.px && g.OW <= 64 && g.W <= 4096 &&
-           hgq_dense_use_bf16_parts(-1) != 0 && (int64_t)g.B * g.OH * g.OW * F * 4 < (1ll << 31) &&
+           (int64_t)g.B * g.OH * g.OW * F * 4 < (1ll << 31) &&
            (int64_t)g.B * g.H * g.W * g.C * 4 < (1ll << 31);
 }
 // rows of a band that fit `pixels` pixels at `width` per row, evened out over the image; the whole image where it fits
@@ -460,11 +460,11 @@ static ThinPlan bwd_plan(const hgq_conv_geom &g) {  // (bands of whole pooling w
 static size_t bwd_lds(int F, const ThinPlan &p) { return (size_t)((F > 32 ? (256 + 32) * 65 : 256 * 33) + 4 * TH_GS + p.patch) * sizeof(float); }
 
 bool conv_thin_fwd_ok(const hgq_conv_geom &g, int F) {
-    if (!thin_shape(g, F)) return false;
+    if (!thin_shape(g, F) || !hgq_dense_use_bf16_parts(-1)) return false;
     const ThinPlan p = thin_plan(g, 128, g.OW, g.OH, 0, 1);
     return p.rows * g.OW <= 128 && thin_patch(g, p, p.rows) * sizeof(float) <= 48 * 1024;
 }
-bool conv_thin_bwd_ok(const hgq_conv_geom &g, int F) {
+bool conv_thin_bwd_shape(const hgq_conv_geom &g, int F) {
     if (!thin_shape(g, F)) return false;
     const ThinPlan p = bwd_plan(g);
     return (p.bands == 1 ? g.OH : p.rows + g.kh - 1) * p.xw <= 256 && bwd_lds(F, p) <= 120 * 1024 && (int64_t)p.rows * g.W * g.C < (1 << 20);

@@ -528,7 +528,7 @@ int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *
 // ---- convolutions.  Pixel indices and places in a window are 32- and 16-bit numbers, tensors below 2 GiB.
 bool conv_parts_shape(const hgq_conv_geom &g, int F) {
     const int lim = 16384;
-    return hgq_dense_use_bf16_parts(-1) != 0 && g.H <= lim && g.W <= lim && g.OH <= lim && g.OW <= lim && g.py <= lim / 2 && g.px <= lim / 2 &&
+    return g.H <= lim && g.W <= lim && g.OH <= lim && g.OW <= lim && g.py <= lim / 2 && g.px <= lim / 2 &&
            (int64_t)g.OH * g.sy <= lim && (int64_t)g.OW * g.sx <= lim && (int64_t)g.kh * g.dly <= lim && (int64_t)g.kw * g.dlx <= lim &&
            (int64_t)g.kh * g.kw * (g.C + 3) < (1 << 20) && (int64_t)g.kh * g.kw * (F + 3) < (1 << 20) && F <= (1 << 16) &&
            (int64_t)g.kh * g.kw * g.C * F * 4 < (1ll << 31) && (int64_t)g.B * g.H * g.W * g.C * 4 < (1ll << 31) &&

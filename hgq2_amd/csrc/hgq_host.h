@@ -65,7 +65,7 @@ int gemm_parts_wgrad(const float *x, const float *dy, const float *mask, float *
 bool dense_split_k(int64_t rows, int K, int F);
 
 // Convolutions of any geometry on the same kernels (the data gradient: unit stride); `splits`: gemm_parts_splits(pixels, K, F).
-bool conv_parts_shape(const hgq_conv_geom &g, int F);
+bool conv_parts_shape(const hgq_conv_geom &g, int F);  // (whichever the matrix instruction)
 int conv_parts_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);
 int conv_parts_dgrad(const float *dy, const float *mask, const float *w, float *dx, const hgq_conv_geom &g, int F, hipStream_t s);
 int conv_parts_wgrad(const float *x, const float *dy, const float *mask, float *part, const hgq_conv_geom &g, int F, int64_t splits, hipStream_t s);
@@ -73,7 +73,7 @@ int conv_parts_wgrad(const float *x, const float *dy, const float *mask, float *
 // Convolutions over few input values per pixel (hgq_conv_thin.hip): which shapes, the bands of rows the backward pass works
 // in, the slices it leaves ([K F + F] each), forward, and data + weight + bias gradient in one pass.
 bool conv_thin_fwd_ok(const hgq_conv_geom &g, int F);
-bool conv_thin_bwd_ok(const hgq_conv_geom &g, int F);
+bool conv_thin_bwd_shape(const hgq_conv_geom &g, int F);  // (whichever the matrix instruction)
 int64_t conv_thin_bwd_tiles(const hgq_conv_geom &g);
 int conv_thin_slices(const hgq_conv_geom &g);
 int conv_thin_fwd(const float *x, const float *w, const float *bias, float *y, const hgq_conv_geom &g, int F, int act, hipStream_t s);
@@ -87,7 +87,7 @@ int conv_patch_launch(int mode, const float *src, const float *mask, const float
 // Weight / bias gradient through LDS-resident operands (3 x 3 and 5 x 5 kernels, unit stride and dilation, channel and
 // filter counts multiples of 4 up to 32, 16-byte aligned operands, bf16-part matrix instruction selected): slices
 // [conv_patch_wgrad_slices][kh kw C F + F] into `part`.
-bool conv_patch_wgrad_ok(const hgq_conv_geom &g, int F);
+bool conv_patch_wgrad_shape(const hgq_conv_geom &g, int F);  // (whichever the matrix instruction)
 int conv_patch_wgrad_slices(const hgq_conv_geom &g, int F);
 int conv_patch_wgrad_launch(const float *x, const float *dy, const float *mask, float *part, const hgq_conv_geom &g, int F, int act,
                             hipStream_t s);

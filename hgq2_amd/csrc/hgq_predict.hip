@@ -216,7 +216,8 @@ static int chain_layout(const hgq_stack_layer *layers, int n, ChainDev &d) {
     return (d.off_a + 2 * CHAIN_BM * CHAIN_LD) * (int)sizeof(float);
 }
 
-// 0: refused, 1: one launch, 2: a launch per layer
+// 0: refused, 1: one launch, 2: a launch per layer (a function of the arguments alone: what hgq_dense_stack_workspace answered
+// holds for the launch, also where another thread has changed the matrix instruction in between)
 static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
     if (!layers || n < 1 || n > HGQ_STACK_MAX_LAYERS || rows < 1) return 0;
     bool chain = true, wide = true, tables = false;
@@ -231,7 +232,6 @@ static int stack_form(const hgq_stack_layer *layers, int n, int64_t rows) {
         tables = tables || (h.iq.i && h.iq.size > h.K) || (h.oq.i && h.oq.size > h.N);
     }
     ChainDev d;
-    wide = wide && hgq_dense_use_bf16_parts(-1) != 0;
     chain = chain && chain_layout(layers, n, d) <= CHAIN_LDS;
     // One launch where the host and the launches are what a call costs, and as long as it is not the slower one on the device
     // either.  Device time of recorded calls, one launch against a launch per layer: 16-64-32-32-5 on 65 536 rows 32 / 54 us,
@@ -284,6 +284,7 @@ using namespace hgq;
 extern "C" int64_t hgq_dense_stack_workspace(const hgq_stack_layer *layers, int n_layers, int64_t rows) {
     const int form = stack_form(layers, n_layers, rows);
     if (form != 2) return form == 1 ? 0 : -1;
+    if (!hgq_dense_use_bf16_parts(-1)) return -1;  // the tiled products know one instruction: layer by layer on the other
     return image_floats(layers, n_layers) + buffer_floats(layers, n_layers, rows, 0) + buffer_floats(layers, n_layers, rows, 1) +
            few_floats(layers, n_layers, rows);
 }

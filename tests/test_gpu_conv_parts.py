@@ -1,6 +1,8 @@
 """Convolutions on the tiled bf16-part products: any channel and filter count, stride, dilation and padding, against 64-bit
 sums, with the bound of two orders of summation (2 (n + 16) 2^-24 of the sum of the products' magnitudes)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -76,3 +78,38 @@ def test_infinities_and_nans_as_on_the_fp32_instruction():
     for a, b in zip(got, want):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isposinf(a), torch.isposinf(b))
         assert torch.equal(torch.isneginf(a), torch.isneginf(b)) and not torch.isfinite(b).all()
+
+
+# the choice of matrix instruction changes between the question for slices and the launch
+@pytest.mark.parametrize('shape,k,F', [((7, 24, 24, 3), 3, 40), ((9, 28, 28, 1), 3, 32), ((5, 11, 11, 16), 3, 32), ((6, 11, 11, 37), 3, 37),
+                                       ((40, 9, 9, 5), 3, 7), ((30, 6, 6, 100), 1, 70), ((3, 12, 12, 4), 3, 8), ((2, 9, 9, 40), 3, 36)])
+@pytest.mark.parametrize('asked', [1, 0])
+def test_slices_hold_when_the_matrix_instruction_changes(shape, k, F, asked):
+    g = torch.Generator().manual_seed(F)
+    geom = ops.conv_geometry(shape, (k, k, shape[-1], F), (1, 1), 'valid', (1, 1))
+    x, w = torch.randn(shape, generator=g), torch.randn((k, k, shape[-1], F), generator=g)
+    dy = torch.randn((shape[0], geom[12], geom[13], F), generator=g)
+    xg, wg, dyg, dx = x.cuda(), w.cuda(), dy.cuda(), torch.empty(shape, device='cuda')
+    lib, desc = _lib.load(), _lib.ConvGeom(*geom)
+    at, stream = ctypes.addressof(desc), torch.cuda.current_stream().cuda_stream
+    before = lib.hgq_dense_use_bf16_parts(asked)
+    try:
+        n, need = lib.hgq_conv2d_bwd_slice_count(at, F), lib.hgq_conv2d_bwd_workspace(at, F)
+        lib.hgq_dense_use_bf16_parts(1 - asked)
+        ws = torch.full((need,), float('nan'), device='cuda')
+        rc = lib.hgq_conv2d_bwd_slices(dyg.data_ptr(), None, xg.data_ptr(), wg.data_ptr(), dx.data_ptr(), ws.data_ptr(), at, F, 0, stream)
+    finally:
+        lib.hgq_dense_use_bf16_parts(before)
+    assert rc == 0
+    width = w.numel() + F
+    total = ws[:n * width].view(n, width).double().sum(0).cpu()
+
+    def exact(xv, wv, dv):
+        xv, wv, bv = xv.clone().requires_grad_(), wv.clone().requires_grad_(), torch.zeros(F, dtype=torch.float64, requires_grad=True)
+        return torch.autograd.grad(_conv64(xv, wv, bv, geom), (xv, wv, bv), dv)
+
+    terms = dy[..., 0].numel()
+    want, size = exact(x.double(), w.double(), dy.double()), exact(x.double().abs(), w.double().abs(), dy.double().abs())
+    for what, got, e, m, count in (('dx', dx, want[0], size[0], k * k * F), ('dw', total[:w.numel()].view(w.shape), want[1], size[1], terms),
+                                   ('db', total[w.numel():], want[2], size[2], terms)):
+        _close(got, e, m, count, what)

@@ -266,3 +266,24 @@ def test_long_contractions_are_split_along_k():
         assert floats(rows, K, N) >= image(K, N) + 2 * rows * N
     for rows, K, N in ((1024, 512, 512), (64, 600, 64), (50000, 2048, 512)):
         assert floats(rows, K, N) == image(K, N)
+
+
+def test_the_answer_for_a_workspace_holds_when_the_matrix_instruction_changes():
+    net = _net((100, 70), bias=False)
+    x = torch.randn((40, 100), generator=torch.Generator().manual_seed(8)).cuda()
+    net(x)
+    lib = _lib.load()
+    descs = (_lib.StackLayer * 1)()
+    assert _stack._layer(net.layers[0], 40, 100, x.device, descs[0], True)
+    with torch.no_grad():
+        want = net(x)
+    floats = lib.hgq_dense_stack_workspace(descs, 1, 40)
+    assert floats > 0
+    y, ws = torch.empty_like(want), torch.empty(floats, device='cuda')
+    before = lib.hgq_dense_use_bf16_parts(0)
+    try:
+        assert lib.hgq_dense_stack_workspace(descs, 1, 40) == -1
+        rc = lib.hgq_dense_stack_predict(descs, 1, x.data_ptr(), y.data_ptr(), 40, ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    finally:
+        lib.hgq_dense_use_bf16_parts(before)
+    assert rc == 0 and torch.equal(y, want)
