@@ -1948,6 +1948,9 @@ extern "C" int hgq_reduce_slices_quant_multi(const hgq_reduce_item *items, int c
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
+// shapes of the tiled products (their lower bound on K is what a wide layer pays off from, not a limit of the kernels)
+static inline bool tiled_shape(int64_t rows, int K, int N) { return gemm_parts_shape(rows, K < 8 ? 8 : K, N); }
+
 static inline int row_parts(int64_t rows, int bm) {
     const int64_t n_tiles = (rows + bm - 1) / bm;
     int g = persistent_grid(n_tiles, 2);
@@ -2033,7 +2036,7 @@ extern "C" int hgq_qdense_fwd(const float *x, const void *k_in, const float *i_i
     }
     // Without a fused input quantizer a width that is not a multiple of four (or an operand off a 16-byte boundary) takes the
     // tiled products of hgq_gemm.hip, which have no alignment rule: 45 930 x 7 x 64 13.7 -> 11.3 us, backward 29.5 -> 16.8 us.
-    if (!quant && g_dense_bf16) return gemm_parts_fwd(x, qw, qb, y, rows, K, N, act, s);
+    if (!quant && g_dense_bf16 && tiled_shape(rows, K, N)) return gemm_parts_fwd(x, qw, qb, y, rows, K, N, act, s);
     const dim3 grid((unsigned)row_parts(rows, FWD_BM), (unsigned)((N + FWD_BN - 1) / FWD_BN));
     if (!quant) {
         hipLaunchKernelGGL((qdense_fwd_kernel<HGQ_TRN, HGQ_WRAP, false>), grid, dim3(256), dyn, s, x, k_in, i_in, f_in, (int64_t)1, qw, qb, y,
@@ -2324,7 +2327,7 @@ static int qdense_bwd_impl(const float *dy, const float *y, const float *x, cons
     }
     if (bcast) return fail(HGQ_ERR_UNSUPPORTED, "hgq_qdense_bwd_mean: K must be a multiple of 4 and x / dx 16-byte aligned");
     const int parts = row_parts(rows, BWD_BM);
-    if (!quant && g_dense_bf16) {  // as in hgq_qdense_fwd
+    if (!quant && g_dense_bf16 && tiled_shape(rows, K, N)) {  // as in hgq_qdense_fwd
         const float *mask = act == HGQ_ACT_RELU ? y : nullptr;
         int rc = gemm_parts_dgrad(dy, mask, qw, dx, rows, K, N, s);
         if (!rc) rc = gemm_parts_wgrad(x, dy, mask, workspace, rows, K, N, parts, s);

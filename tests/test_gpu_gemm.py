@@ -76,3 +76,16 @@ def test_infinities_and_nans_as_on_the_fp32_instruction():
     for a, b in zip(got, want):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isposinf(a), torch.isposinf(b))
         assert torch.equal(torch.isneginf(a), torch.isneginf(b)) and not torch.isfinite(b).all()
+
+
+def test_contractions_beyond_the_tiled_products():
+    # more inputs than the tiled products state: the general dense kernel
+    g = torch.Generator().manual_seed(9)
+    rows, K, N = 3, 2**20 + 3, 2
+    x, w = _operand(g, (rows, K), 3).cuda(), _operand(g, (K, N), 3).cuda()
+    y = torch.empty((rows, N), device='cuda')
+    rc = _lib.load().hgq_qdense_fwd(x.data_ptr(), None, None, None, 0, w.data_ptr(), None, y.data_ptr(), None, rows, K, N, 0, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    xd, wd = x.double().cpu(), w.double().cpu()
+    _close(y, xd @ wd, xd.abs() @ wd.abs(), K, 'forward')
