@@ -89,3 +89,15 @@ def test_contractions_beyond_the_tiled_products():
     assert rc == 0
     xd, wd = x.double().cpu(), w.double().cpu()
     _close(y, xd @ wd, xd.abs() @ wd.abs(), K, 'forward')
+
+
+def test_data_gradient_in_large_tiles():
+    # 384 tiles of 128 x 128 for the data gradient, both sides ragged
+    g = torch.Generator().manual_seed(10)
+    rows, K, N = 49100, 100, 70
+    x, w = _operand(g, (rows, K), 3).cuda().requires_grad_(), _operand(g, (K, N), 10).cuda()
+    dy = torch.randn((rows, N), generator=g).cuda()
+    y = ops.matmul_bias_act(x, w, None, 1)
+    (gx,) = torch.autograd.grad(y, (x,), dy)
+    dz, wd = dy.double().cpu() * (y.detach().cpu() > 0), w.double().cpu()
+    _close(gx, dz @ wd.T, dz.abs() @ wd.abs().T, N, 'data gradient')
