@@ -469,7 +469,10 @@ __global__ void ebops_finish_bwd_kernel(const float *g, const float *beta, float
 // the order in which they arrive, so the loss is the same in every run and in every replay of a recorded step (a float
 // atomic would round differently with every arrival order).  state == NULL: a single workgroup, no meeting at all.
 #define CE_FIX 1099511627776.0f  // 2^40: a sum of up to 2^22 in magnitude keeps 2^-40 resolution in 63 bits
-#define CE_REGS 16  // classes whose row fits the registers of its thread
+// REGS: classes whose row fits that many registers of its thread (0: any number, from memory).  The row and its label are then
+// asked for together and every exponential is taken once, the same operations in the same order: 4096 x 10 8.8 -> 6.7 us,
+// 262 144 x 16 84 -> 40 us.  As few registers as do: two classes in sixteen took 10 % longer than from memory.
+template <int REGS>
 __global__ __launch_bounds__(256) void sparse_ce_kernel(const float *__restrict__ logits,
                                                         const int64_t *__restrict__ labels, float *loss,
                                                         float *__restrict__ dlogits, int64_t rows, int C, uint32_t *state) {
@@ -478,20 +481,18 @@ __global__ __launch_bounds__(256) void sparse_ce_kernel(const float *__restrict_
     float acc = 0.0f;
     for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < rows; r += (int64_t)gridDim.x * 256) {
         const float *z = logits + r * C;
-        if (C <= CE_REGS) {
-            // the row and its label asked for together, every exponential taken once (same operations in the same order as
-            // below): 4096 x 10 10.5 -> 7.3 us
+        if (REGS) {
             const int64_t lab = labels[r];
-            float v[CE_REGS];
+            float v[REGS ? REGS : 1];
 #pragma unroll
-            for (int c = 0; c < CE_REGS; ++c) v[c] = z[c < C ? c : 0];
+            for (int c = 0; c < REGS; ++c) v[c] = z[c < C ? c : 0];
             float mx = v[0];
 #pragma unroll
-            for (int c = 1; c < CE_REGS; ++c) mx = c < C ? fmaxf(mx, v[c]) : mx;
+            for (int c = 1; c < REGS; ++c) mx = c < C ? fmaxf(mx, v[c]) : mx;
             const bool lab_ok = (uint64_t)lab < (uint64_t)C;
             float se = 0.0f, zl = 0.0f;
 #pragma unroll
-            for (int c = 0; c < CE_REGS; ++c) {
+            for (int c = 0; c < REGS; ++c) {
                 if (c < C) {
                     zl = c == lab ? v[c] - mx : zl;
                     v[c] = expf(v[c] - mx);
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(256) void sparse_ce_kernel(const float *__restrict_
                 float *d = dlogits + r * C;
                 const float inv = 1.0f / se;
 #pragma unroll
-                for (int c = 0; c < CE_REGS; ++c)
+                for (int c = 0; c < REGS; ++c)
                     if (c < C) d[c] = lab_ok ? (v[c] * inv - (c == lab ? 1.0f : 0.0f)) * inv_rows : 0.0f;
             }
             continue;
@@ -838,7 +839,12 @@ extern "C" int hgq_sparse_ce_fwd_bwd(const float *logits, const int64_t *labels,
     hipStream_t s = (hipStream_t)stream;
     if (state && ((uintptr_t)state & 7u)) return fail(HGQ_ERR_ARG, "hgq_sparse_ce_fwd_bwd: state must be 8-byte aligned");
     const int grid = state ? persistent_grid((rows + 255) / 256, 4) : 1;
-    hipLaunchKernelGGL(sparse_ce_kernel, dim3(grid), dim3(256), 0, s, logits, labels, loss, dlogits, rows, C, state);
+#define HGQ_CE(REGS) hipLaunchKernelGGL(sparse_ce_kernel<REGS>, dim3(grid), dim3(256), 0, s, logits, labels, loss, dlogits, rows, C, state)
+    if (C <= 4) HGQ_CE(4);
+    else if (C <= 8) HGQ_CE(8);
+    else if (C <= 16) HGQ_CE(16);
+    else HGQ_CE(0);
+#undef HGQ_CE
     return check_launch("hgq_sparse_ce_fwd_bwd");
 }
 
