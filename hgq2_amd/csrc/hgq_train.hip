@@ -201,12 +201,13 @@ __global__ __launch_bounds__(HGQ_EBOPS_NT) void dense_ebops_multi_kernel(DenseEb
 }
 
 // Mean squared error: per-workgroup partial sums (fixed order inside a workgroup), added in order
-// by one wavefront of a second launch: the loss does not depend on scheduling.
+// by one workgroup of a second launch: the loss does not depend on scheduling.
 #define MSE_PARTS 2048
 // dpred (may be null): also receives the gradient for a unit upstream gradient, (pred - target) * two_over_n, the value
 // mse_bwd_kernel gives for g = 1
-// NT: operands beyond the 256 MB memory-side cache, which the next launch could not find there anyway.  805 MB (67 Mi values): 154 us =
-// 5.2 TB/s, what streams of this size reach on this card (four workgroups per CU, cached: 170 us).
+// NT: past the 256 MB memory-side cache.  It pays where the gradient alone fills that cache, so that the launch that reads it
+// next could not find it there: this launch and a reader of the gradient, cached against not, 2^26 values 214 / 199 us, 2^25
+// 93 / 98 us, 2^24 47 / 52 us.  2^26 values (805 MB) alone: 144 us = 5.6 TB/s (four workgroups per CU, cached: 163 us).
 template <bool NT>
 __global__ __launch_bounds__(256) void mse_partial_kernel(const float *__restrict__ pred, const float *__restrict__ target, int64_t n,
                                                           float *__restrict__ part, float *__restrict__ dpred, float two_over_n) {
@@ -987,7 +988,7 @@ extern "C" int hgq_mse_fwd_bwd(const float *pred, const float *target, float *lo
     hipStream_t s = (hipStream_t)stream;
     int grid = persistent_grid(((n >> 2) + 255) / 256, 8);
     if (grid > MSE_PARTS) grid = MSE_PARTS;
-    if (n > (1 << 24))
+    if (n >= (1 << 26))
         hipLaunchKernelGGL(mse_partial_kernel<true>, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, dpred, 2.0f / (float)n);
     else
         hipLaunchKernelGGL(mse_partial_kernel<false>, dim3(grid), dim3(256), 0, s, pred, target, n, workspace, dpred, 2.0f / (float)n);
