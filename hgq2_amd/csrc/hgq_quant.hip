@@ -1074,27 +1074,28 @@ extern "C" int hgq_quantize_bwd_multi(const hgq_quant_grad_item *items, int coun
 }
 
 // Geometry of the per-column backward for the sliced form of the bit-width gradients.
-static bool sliced_bwd_geometry(int64_t n, int64_t bw_size, int64_t bw_inner, bool &vec, int &TX, int64_t &gx, int64_t &gy, int64_t &rows_per_wg) {
+static bool sliced_bwd_geometry(int64_t n, int64_t bw_size, int64_t bw_inner, bool &vec, int &TX, int64_t &gx, int64_t &gy) {
     if (n < 1 || bw_size < 2 || bw_inner != 1 || bw_size >= n || n % bw_size != 0 || bw_size * 4 * 256 * QC_U >= (1ll << 31)) return false;
     vec = bw_size % 4 == 0;
     const int64_t cg = vec ? bw_size / 4 : bw_size;
     TX = pow2_floor_le64(cg);
     gx = (cg + TX - 1) / TX;
+    int64_t rows_per_wg;  // (the kernel deals its batches out in turn)
     return cols_grid(n / bw_size, bw_size, (256 / TX) * QC_U, gx, gy, rows_per_wg);
 }
 
 extern "C" int64_t hgq_quantize_bwd_workspace(int64_t n, int64_t bw_size, int64_t bw_inner) {
     bool vec;
     int TX;
-    int64_t gx, gy, rows_per_wg;
-    return sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy, rows_per_wg) ? gy * 2 * bw_size : 0;
+    int64_t gx, gy;
+    return sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy) ? gy * 2 * bw_size : 0;
 }
 
 extern "C" int64_t hgq_quantize_bwd_slice_count(int64_t n, int64_t bw_size, int64_t bw_inner) {
     bool vec;
     int TX;
-    int64_t gx, gy, rows_per_wg;
-    return sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy, rows_per_wg) ? gy : 0;
+    int64_t gx, gy;
+    return sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy) ? gy : 0;
 }
 
 static int quantize_bwd_sliced_impl(const float *dy, const float *x, const void *k, const float *i, const float *fb, float *dx,
@@ -1121,8 +1122,8 @@ static int quantize_bwd_sliced_impl(const float *dy, const float *x, const void 
     hipStream_t s = (hipStream_t)stream;
     bool vec;
     int TX;
-    int64_t gx, gy, rows_per_wg;
-    if (!sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy, rows_per_wg))
+    int64_t gx, gy;
+    if (!sliced_bwd_geometry(n, bw_size, bw_inner, vec, TX, gx, gy))
         return fail(HGQ_ERR_UNSUPPORTED, "hgq_quantize_bwd_sliced: shape outside the per-column kernels (hgq_quantize_bwd_workspace returns 0 for it)");
     if (!dy || !x || !k || !i || !fb || !dfb || !workspace) return fail(HGQ_ERR_ARG, "hgq_quantize_bwd_sliced: null pointer");
     const Mode m(mode);

@@ -107,7 +107,7 @@ def dense_contraction(x, iq, qkernel2d, qbias1d, act_name, training, oq=None, ou
     if fused_bwd:
         y, _ = ops.qdense(x2d, None, None, None, qkernel2d, qbias1d, act_code, 0, 0, False)
         return y, act_code != _lib.ACT_NONE, None, False
-    # shapes beyond the fused backward kernel: the implicit-GEMM kernels in their 1 x 1 form
+    # shapes beyond the fused backward kernel: convolutions in their 1 x 1 form (tiled products for the most part)
     y = ops.matmul_bias_act(x2d, qkernel2d, qbias1d, act_code)
     return y, act_code != _lib.ACT_NONE, None, False
 

@@ -2592,7 +2592,8 @@ def conv2d(xq: Tensor, qw: Tensor, qb, strides=(1, 1), padding='valid', dilation
 
 
 def matmul_bias_act(x2d: Tensor, qw: Tensor, qb, act: int = 0) -> Tensor:
-    """``act(x2d @ qw + qb)`` for any K, N: the 1 x 1 case of the implicit-GEMM kernels."""
+    """``act(x2d @ qw + qb)`` for any K, N: the 1 x 1 case of a convolution (tiled products, few columns and long contractions
+    split along K)."""
     rows, K = x2d.shape
     N = qw.shape[1]
     geom = (rows, 1, 1, K, 1, 1, 1, 1, 0, 0, 1, 1, 1, 1)
