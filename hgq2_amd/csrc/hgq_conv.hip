@@ -1696,7 +1696,10 @@ extern "C" int hgq_conv2d_fwd(const float *xq, const float *qw, const float *qb,
     }
     if (nz == 1 && conv_thin_fwd_ok(*g, F)) return conv_thin_fwd(xq, qw, qb, y, *g, F, act, s);
     if (nz == 1 && aligned16(xq) && conv_patch_ok(0, *g, F)) return conv_patch_launch(0, xq, nullptr, qw, qb, y, *g, F, act, s);
-    // (300 x 11 x 11, 3 x 3, 40 -> 40: 22 -> 15 us; 1024 x 13 x 13, 37 -> 37: 135 -> 51 us against the implicit GEMM below)
+    // Any other geometry: the tiled products, 1.2 - 2.8 x the implicit GEMM below over depths of 5 - 256, strides and dilations of
+    // 1 and 2, 1 x 1 to 7 x 7 (300 x 11 x 11, 3 x 3, 40 -> 40 21.9 -> 15.2 us; 1024 x 13 x 13, 64 -> 64 104 -> 68 us; 300 x 16 x 16,
+    // stride 2, 128 -> 128 87 -> 56 us).  One to three channels at stride 2 are the exception, 9.4 - 10.4 -> 10.3 - 11.2 us on 300
+    // images of 24 x 24, and 34 -> 28 us on 1024 of 28 x 28.
     if (nz == 1 && parts_on() && conv_parts_shape(*g, F)) return conv_parts_fwd(xq, qw, qb, y, *g, F, act, s);
     const bool vec = g->C % 4 == 0 && aligned16(xq) && (int64_t)g->B * g->H * g->W * g->C * 4 < (1ll << 31);
     if (F <= 32) {
@@ -1812,7 +1815,7 @@ static int conv2d_bwd_impl(const float *dy, const float *y, const float *xq, con
 #undef HGQ_DG
         } else if (aligned16(dy) && (!mask || aligned16(mask)) && conv_patch_ok(1, *g, F)) {
             if ((rc = conv_patch_launch(1, dy, mask, qw, nullptr, dxq, *g, F, act, s))) return rc;
-        } else if (g->sy == 1 && g->sx == 1 && parts && conv_parts_shape(*g, F)) {  // 300 x 11 x 11, 3 x 3, 40 -> 40: 50 -> 27 us
+        } else if (g->sy == 1 && g->sx == 1 && parts && conv_parts_shape(*g, F)) {  // (over the same range 1.3 - 3.5 x; 300 x 11 x 11, 3 x 3, 40 -> 40: 48 -> 26 us)
             if ((rc = conv_parts_dgrad(dy, act == HGQ_ACT_RELU ? mask : nullptr, qw, dxq, *g, F, s))) return rc;
         } else {
             const bool vec = F % 4 == 0 && aligned16(dy) && (!mask || aligned16(mask)) && rows * F * 4 < (1ll << 31);

@@ -14,9 +14,10 @@
 // all finite is contracted on the fp32 instruction.)  A row of dZ is owned (for dW) by one band; the rows above it are
 // contracted again for G, which costs a quarter of the matrix work and no memory traffic beyond L2.
 //
-// 300 x 24 x 24 x 3 onto 40 filters of 3 x 3: backward 26 us (47 MB; gathered kernels for the two gradients 77 + 72 us), forward
-// 12.6 us (implicit GEMM 30 us).  1024 x 28 x 28 x 1 onto 32, behind a pooling: backward 52 us (multiply-adds per pixel and
-// filter 54 us).  Bound by vector instructions: about 400 per wavefront and band for staging, splitting and the nine taps.
+// 300 x 24 x 24 x 3 onto 40 filters of 3 x 3: backward 30 us with its reduction (47 MB; gathered kernels for the two gradients
+// 150 us), forward 11.6 us (implicit GEMM 26 us).  1024 x 28 x 28 x 1 onto 32, behind a pooling: backward 54 us (multiply-adds per
+// pixel and filter 57 us; few filters or wide rows are theirs, see thin_bwd_shape).  Bound by vector instructions, 50 for every
+// matrix instruction: staging, splitting and the nine taps.
 #include "hgq_device.h"
 #include "hgq_host.h"
 

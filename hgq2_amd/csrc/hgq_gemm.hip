@@ -17,10 +17,12 @@
 // from the low bits of its values (quantized operands of up to 8 bits: one part each, one matrix instruction per product);
 // gradients are arbitrary fp32 numbers and always take three.
 //
-// What bounds them: 50 000 x 256 onto 512 (153 MB, 13 GFLOP) takes 76 us, 50 000 x 512 onto 256 57 us (implicit GEMM: 174 and
-// 160 us) - 2 TB/s and 170 - 230 TFLOP/s, in between the two roofs: the chain load -> agree -> stage -> multiply of a tile step,
-// hidden by the second workgroup of a CU alone.  4096 x 256 x 512: forward 10.8, data gradient 15.9, weight gradient 13.4 us
-// (16.8, 25.5, 16.2 us).
+// What bounds them: 50 000 x 256 onto 512 (153 MB, 13 GFLOP) takes 56 us, 50 000 x 512 onto 256 47 us (implicit GEMM: 167 and
+// 153 us) - 3 TB/s and 240 - 280 TFLOP/s, in between the two roofs: the chain load -> agree -> stage -> multiply of a tile step,
+// hidden by the second workgroup of a CU alone (matrix cores busy 8 % of the time, wavefronts waiting 47 %; 22 vector
+// instructions per matrix instruction).  4096 x 256 x 512: forward 9.4, data gradient 14.5, weight gradient 20.8 us with its
+// reduction (16.6, 34.3, 24.7 us).  Below some 300 rows the weight gradient is 0.7 - 1 us behind the gathered kernel it
+// replaced (256 x 256 x 512 15.0 / 14.0 us); the data gradient beside it is 20 us ahead.
 #include "hgq_device.h"
 #include "hgq_host.h"
 
@@ -479,6 +481,8 @@ static void gp_launch(GpArgs g, int splits, hipStream_t s) {
 
 // Tile of a product with `m` x `n` outputs.  128 x 128 tiles split and stage each operand value half as often, but a launch
 // needs two of them per CU to cover the staging of one with the products of the other; fewer outputs go to 64 x 64 tiles.
+// 64 x 64 against 128 x 128, forward: 4096 x 256 -> 512 (128 large tiles) 9.8 / 15.2 us, 8192 x 256 -> 512 (256) 16.7 / 16.7 us,
+// 12 288 x 256 -> 512 (384) 23.0 / 18.3 us, 32 768 x 256 -> 512 (1024) 53.4 / 32.7 us; data gradients have the same line.
 template <int OP>
 static void gp_dispatch(const GpArgs &g, int64_t m, int64_t n, int splits, hipStream_t s) {
     const int64_t big = ((m + 127) / 128) * ((n + 127) / 128) * splits;

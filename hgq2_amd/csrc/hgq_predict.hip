@@ -9,8 +9,8 @@
 //   launch per quantizer and contraction, sixteen in all: 512 us).
 // * Wider layers, or many rows: one launch quantizes all kernels and biases into the workspace, one the input; then per layer
 //   a tiled product whose epilogue applies the next layer's input quantizer (a pass over [rows, N] each way less), the
-//   streaming kernel of up to 64 x 64, or what hgq_conv2d_fwd has for a product of few tiles.  50 000 rows through 256-512-256-128-10: 195 us (a launch per quantizer and
-//   contraction: 484 us).
+//   streaming kernel of up to 64 x 64, or what hgq_conv2d_fwd has for a product of few tiles.  50 000 rows through
+//   256-512-256-128-10: 195 us (a launch per quantizer and contraction: 484 us).
 //
 // Arithmetic per value is that of hgq_quantize_fwd and of the layer's own contraction; the variables are quantized again on
 // every call (they may have been written in between).
