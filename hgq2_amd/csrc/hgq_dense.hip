@@ -1749,9 +1749,7 @@ __global__ __launch_bounds__(256, 2) void dense_moments_bwd_gram_kernel(const fl
 }
 
 // out[e] = sum over slices of part[g][e], in slice order.  256 threads = 64 elements x 4 slice groups.
-// a joint reduction gives a workgroup 256 entries instead of 64 of a set of few slices and many entries
-#define RP_FEW 64      // (whole multiple of RP_G)
-#define RP_WIDE 32768
+#define RP_FEW 64  // slices up to which a joint reduction may give a workgroup 256 entries instead of 64 (whole multiple of RP_G)
 #define RP_G 16  // slice groups per entry: 64 entries x 16 groups = 1024 threads, few dependent load batches per thread
 __global__ __launch_bounds__(64 * RP_G) void reduce_parts_kernel(const float *__restrict__ part, int n_parts, int64_t M,
                                                                  float *dqw, int64_t n_dqw, float *dqb, int64_t n_dqb,
@@ -1811,13 +1809,11 @@ struct ReduceQuants {
     int8_t attach[HGQ_REDUCE_BATCH][3];
 };
 
-// Sets of few slices and many entries (wide layers: 131 072 entries x 16): 256 entries x 4 quads of groups per workgroup, so
-// that more than a sixteenth of the threads write and run the quantizers' backward, and a thread has up to sixteen loads in
-// flight.  All slices of a 256-512-256-128-10 step: 14.4 -> 10.0 us.  Same association of the sums either way.
-__host__ __device__ static inline bool rp_few(const hgq_reduce_item &it) { return it.n_slices <= RP_FEW && it.width > RP_WIDE; }
-
-// FEW: the launch holds such a set (a launch that does not is 0.5 - 0.9 us faster without the second form in its code: 512
-// slices of 1088 entries 4.1 against 4.8 us)
+// FEW: sets of few slices (wide layers: 131 072 entries x 16) by 256 entries x 4 quads of groups per workgroup, so that more than
+// a sixteenth of the threads write and run the quantizers' backward, and a thread has up to sixteen loads in flight.  Same
+// association of the sums either way.  It pays in launches of more workgroups than the card holds at once (two per CU): all
+// slices of a 256-512-256-128-10 step 14.4 -> 10.0 us, of an image network's (3 slices of 32 410 entries its widest set) 10.2 -> 7.6 us;
+// 512 slices of 1088 entries 4.1 -> 4.8 us, 64 of 20 000 3.7 -> 4.3 us, with both forms in the kernel's code.
 template <bool QUANTS, bool FEW>
 __global__ __launch_bounds__(64 * RP_G) void reduce_parts_multi_kernel(const ReduceBatch b, const ReduceQuants q) {
     __shared__ float red[64 * RP_G];
@@ -1828,7 +1824,7 @@ __global__ __launch_bounds__(64 * RP_G) void reduce_parts_multi_kernel(const Red
     const int n_parts = it.n_slices;
     const int64_t M = it.width;
     const int per = (n_parts + RP_G - 1) / RP_G;
-    const bool few = FEW && rp_few(it);
+    const bool few = FEW && n_parts <= RP_FEW;
     const int cols = few ? 256 : 64, e_local = threadIdx.x & (cols - 1), grp = threadIdx.x / cols;
     const int64_t e = (int64_t)((int)blockIdx.x - b.first_block[t]) * cols + e_local;
     float s = 0.f;
@@ -1924,7 +1920,9 @@ static int reduce_slices_impl(const hgq_reduce_item *items, int count, const hgq
             q.item[nq++] = quants[j];
         }
         int64_t blocks = 0;
-        bool few = false;
+        for (int t = 0; t < b.count; ++t) blocks += items[base + t].width > 0 ? (items[base + t].width + 63) / 64 : 0;
+        const bool few = blocks > persistent_grid(1 << 30, 2);
+        blocks = 0;
         for (int t = 0; t < b.count; ++t) {
             const hgq_reduce_item &it = items[base + t];
             if (it.n_slices < 1 || it.width < 1 || !it.slices) return fail(HGQ_ERR_ARG, "%s: bad sizes in item %d", who, base + t);
@@ -1932,8 +1930,7 @@ static int reduce_slices_impl(const hgq_reduce_item *items, int count, const hgq
                 return fail(HGQ_ERR_ARG, "%s: item %d: output lengths do not add up to the slice width", who, base + t);
             b.item[t] = it;
             b.first_block[t] = (int)blocks;
-            few = few || rp_few(it);
-            blocks += rp_few(it) ? (it.width + 255) / 256 : (it.width + 63) / 64;
+            blocks += few && it.n_slices <= RP_FEW ? (it.width + 255) / 256 : (it.width + 63) / 64;
             if (blocks > (1 << 24)) return fail(HGQ_ERR_UNSUPPORTED, "%s: too many columns", who);
         }
         for (int t = b.count; t <= HGQ_REDUCE_BATCH; ++t) b.first_block[t] = (int)blocks;
