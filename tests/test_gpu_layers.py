@@ -620,6 +620,43 @@ def test_dense_backward_in_two_halves_gives_the_same_bits(dev):
         ops.reduce_slices_multi_op(slices[:1], outs[:2] + [outs[5]], skip[:3])  # lengths do not add up to the width
 
 
+@pytest.mark.parametrize('quants', [False, True])
+def test_joint_reduction_in_a_large_launch_gives_the_same_bits(dev, quants):
+    """Sets of few and of many slices, widths around a workgroup's 64 and 256 entries, in one launch that fits the card (each set
+    alone) and in one of more workgroups than two per CU (all of them): identical sums, and identical gradients of a quantizer
+    behind a segment."""
+    from hgq2_amd import _lib, ops
+
+    g = torch.Generator().manual_seed(17)
+    shapes = [(1, 255), (3, 256), (16, 257), (17, 64), (64, 513), (65, 300), (130, 1088), (5, 140001)]
+    slices = [torch.randn(s, generator=g).to(dev) for s in shapes]
+    cut = [(m // 2, m - m // 2 - m // 5, m // 5) for _, m in shapes]
+    xs = [(torch.randn(c[0], generator=g) * 3).to(dev) for c in cut]
+    ks = [torch.ones(c[0], dtype=torch.uint8, device=dev) for c in cut]
+    is_ = [torch.randint(-1, 4, (c[0],), generator=g).float().to(dev) for c in cut]
+    fs = [torch.randint(0, 7, (c[0],), generator=g).float().to(dev) for c in cut]
+    mode = _lib.mode_bits('RND', 'SAT', training=True, round_params=True)
+
+    def run(sets):
+        outs = [torch.full((n,), 7.0, device=dev) for t in sets for n in cut[t]]
+        args = ([slices[t] for t in sets], outs, [False] * len(outs))
+        if not quants:
+            ops.reduce_slices_multi_op(*args)
+            return [outs[3 * j:3 * j + 3] for j in range(len(sets))]
+        n = len(sets)
+        got = ops.reduce_slices_quant_multi_op(*args, *([v[t] for t in sets] for v in (xs, ks, is_, fs)), [mode] * n, list(range(n)), [0] * n)
+        return [outs[3 * j:3 * j + 3] + got[j::n] for j in range(n)]
+
+    together = run(range(len(shapes)))
+    for t, (n, m) in enumerate(shapes):
+        if m <= 64 * 512:  # (512 workgroups on 256 CUs: the last set alone is a large launch too)
+            for a, b in zip(together[t], run([t])[0]):
+                assert torch.equal(a, b), shapes[t]
+        exact, size = slices[t].double().sum(0), slices[t].double().abs().sum(0)
+        err = (torch.cat(together[t][:3]).double() - exact).abs()
+        assert bool((err <= 2 * n * 2.0**-24 * size).all()), shapes[t]  # n additions in any order: at most n u / (1 - n u)
+
+
 def test_fused_stack_sees_updates_made_by_the_per_layer_optimizer(dev):
     """Alternating the whole-step kernels with the per-layer path: the fused trainer must not reuse the quantized
     weight image of its previous step after ``SGD.step`` (which writes through ``.data``) changed the variables."""
